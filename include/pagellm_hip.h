@@ -74,7 +74,8 @@ int plh_create(plh_ctx** out, int device);
 void plh_destroy(plh_ctx* ctx);
 const char* plh_last_error(const plh_ctx* ctx);
 /* Queue work on `stream` (a hipStream_t, e.g. torch's current stream); NULL
- * restores the context's own stream.  Moving to another stream records an
+ * restores the context's own stream (a blocking stream, ordered with the
+ * device's default stream in both directions).  Moving to another stream records an
  * event on the stream being left that closes the calls queued there; the
  * next call on the new stream waits for it (calls on one stream record
  * nothing).  A stream stays in use until the context moves off it or is

@@ -259,7 +259,11 @@ int plh_create(plh_ctx** out, int device) {
   int rc = PLH_OK;
   do {
     if (hipSetDevice(device) != hipSuccess) { rc = PLH_ERR_HIP; break; }
-    if (hipStreamCreateWithFlags(&c->own_stream, hipStreamNonBlocking) != hipSuccess) { rc = PLH_ERR_HIP; break; }
+    // a blocking stream: ordered with the device's default stream, so a caller
+    // whose tensors are made on the default stream (torch's current stream
+    // outside any `with torch.cuda.stream`, whose handle is null) needs no
+    // synchronisation of its own
+    if (hipStreamCreateWithFlags(&c->own_stream, hipStreamDefault) != hipSuccess) { rc = PLH_ERR_HIP; break; }
     c->stream = c->own_stream;
     if (hipMalloc(&c->fallback, sizeof(unsigned long long)) != hipSuccess) { rc = PLH_ERR_OUT_OF_MEMORY; break; }
     if (hipMemset(c->fallback, 0, sizeof(unsigned long long)) != hipSuccess) { rc = PLH_ERR_HIP; break; }

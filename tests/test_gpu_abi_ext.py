@@ -351,3 +351,26 @@ def test_workspace_users_interleaved_on_streams():
     finally:
         c.set_stream(None)
         c.close()
+
+
+def test_default_stream_work_is_ordered():
+    """Torch's default stream has a null handle, which selects the context's
+    own stream: tensors still being written on the default stream are read
+    only once they are complete, and what the default stream does next sees
+    the results."""
+    import torch
+
+    from pagellm_amd.head import LogitsHead
+
+    D, V = 512, 128256
+    head = LogitsHead(np.ones(D, np.float32), np.zeros((D, V), np.float32))
+    h = torch.ones((16, D), device="cuda")
+    out = torch.empty((16, V), device="cuda")
+    busy = torch.randn((4096, 4096), device="cuda")
+    for i in (1, 2, 3):
+        out.fill_(-1.0)
+        for _ in range(20):
+            busy = (busy @ busy).clamp_(-1, 1)
+        head.lm_head.fill_(float(i))  # queued behind the products
+        got = head(h, out=out).clone()  # the copy, too, is on the default stream
+        torch.testing.assert_close(got, torch.full_like(got, i * D * (1 + 1e-5) ** -0.5), rtol=1e-5, atol=0)
