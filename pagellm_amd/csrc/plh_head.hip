@@ -8,6 +8,8 @@
 //                   once);
 //   k_head_act      act = (h * r) * norm, stored k-major and zero-padded to
 //                   whole tiles (32 in k, 256 in n);
+//   k_head_prep,    the same for at most 32 rows (see "few rows" below);
+//   k_head_skinny
 //   k_head_gemm     out = act @ W on the fp32 matrix cores
 //                   (v_mfma_f32_32x32x2_f32, products and sums in float32).
 //                   A workgroup of 8 waves (two per SIMD) owns a 256-row x
@@ -269,11 +271,244 @@ k_head_gemm(HeadArgs a) {
   else head_tile<false, false>(a, sm);
 }
 
+// ------------------------------------------------------------- few rows
+//
+// Up to 32 rows (a decode step of a few sequences) the product is bound by
+// one read of W from HBM, and a 256-row tile spends its time multiplying
+// padding.  These rows take two launches of their own: k_head_prep (RMSNorm
+// and the operand layout, one workgroup per row) and k_head_skinny.
+//
+// k_head_skinny<R>: R = 16 or 32 rows x 128 columns per workgroup on
+// v_mfma_f32_16x16x4 / 32x32x2_f32.  The 8 waves share the columns and split
+// k, so that a workgroup has 8 independent streams of W in flight; W goes
+// from HBM straight into the MFMA operand registers (a lane's 16-byte load is
+// one k row's value for each of four column tiles whose columns interleave by
+// 4), with no LDS on the way, and the waves' sums meet in LDS once at the
+// end, in a fixed order.  A lane's columns 4c .. 4c+3 are the same lane's of
+// four accumulators, so the logits leave in 16-byte stores.
+//
+// 8 x 4096 x 128 256: 370 us, W read at 5.7 TB/s (a large copy moves 5.2 TB/s
+// here); 2 000 us in the 256-row tile.
+
+// k values per operand group: one 16-byte load of act per lane
+template <int R>
+struct Skinny {
+  static constexpr int kQ = 64 / R;          // k values side by side in one MFMA
+  static constexpr int kG = 4 * kQ;          // k values per group (4 MFMA steps)
+  static constexpr int kCG = 128 / (4 * R);  // column groups of 4 R columns
+};
+constexpr int kSkinnyCols = 128;
+
+__host__ __device__ constexpr int skinny_rows(int N) { return N <= 16 ? 16 : 32; }
+__host__ __device__ constexpr int skinny_groups(int D, int R) { return (D + 256 / R - 1) / (256 / R); }
+
+// act for k_head_skinny: group g holds k = g*kG .. +kG; lane (q, row) of an
+// MFMA step t reads k = g*kG + kQ*t + q, so its four steps are 16 bytes at
+// ((g*kQ + q)*R + row)*4.  Zero outside d < D; rows N .. R-1 are not written
+// (an accumulator row depends on its own act row only, and those rows of the
+// accumulators are never stored).
+template <int R>
+__global__ __launch_bounds__(kThreads) void k_head_prep(HeadArgs a) {
+  using S = Skinny<R>;
+  __shared__ double red[kWaves];
+  const int n = blockIdx.x, D = a.D;
+  const float* x = a.h + (size_t)n * a.ldh;
+  double s = 0.0;
+  for (int d = threadIdx.x; d < D; d += kThreads) {
+    const float v = x[d];
+    s += (double)(v * v);  // the float32 square, as numpy forms x * x
+  }
+  s = block_sum(s, red);
+  // as in k_head_rms, by every thread alike
+  const float r = 1.0f / sqrtf((float)s / (float)D + a.eps);
+  const int Dp = skinny_groups(D, R) * S::kG;
+  for (int d = threadIdx.x; d < Dp; d += kThreads) {
+    const int g = d / S::kG, e = d % S::kG;
+    a.act[((size_t)(g * S::kQ + e % S::kQ) * R + n) * 4 + e / S::kQ] = d < D ? (x[d] * r) * a.norm[d] : 0.0f;
+  }
+}
+
+typedef float f32x4u __attribute__((ext_vector_type(4))) __attribute__((aligned(4)));
+
+template <int R>
+struct SkinnyAcc;
+template <>
+struct SkinnyAcc<16> {
+  typedef f32x4 T;
+  static __device__ __forceinline__ T mma(float x, float y, T c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(x, y, c, 0, 0, 0);
+  }
+  // accumulator register r of lane l holds this row
+  static __device__ __forceinline__ int row(int r, int l) { return 4 * (l >> 4) + r; }
+};
+template <>
+struct SkinnyAcc<32> {
+  typedef f32x16 T;
+  static __device__ __forceinline__ T mma(float x, float y, T c) {
+    return __builtin_amdgcn_mfma_f32_32x32x2f32(x, y, c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ int row(int r, int l) { return 8 * (r >> 2) + 4 * (l >> 5) + (r & 3); }
+};
+
+// ANY: V < 128, or rows of W more than 64 MB apart: columns are read one by
+// one and clamped.  Otherwise the last workgroup's columns are the last 128,
+// so every 16-byte load lies inside its row (columns of two workgroups are
+// computed alike by both), and the loads are buffer loads whose row offsets
+// are scalars.
+template <int R, bool ANY>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) void k_head_skinny(HeadArgs a) {
+  using S = Skinny<R>;
+  using A = SkinnyAcc<R>;
+  constexpr int kRegs = R * R / 64;
+  // half of the waves' accumulators at a time
+  __shared__ f32x4 sm[kWaves / 2][S::kCG * kRegs][64];
+  const int D = a.D, V = a.V, l = lane(), w = uniform(wave());
+  const int v0 = ANY ? (int)blockIdx.x * kSkinnyCols : min((int)blockIdx.x * kSkinnyCols, V - kSkinnyCols);
+  const int c = l % R, q = l / R;
+  const float* act = a.act + (size_t)(q * R + c) * 4;
+
+  typename A::T acc[S::kCG][4];
+#pragma unroll
+  for (int cg = 0; cg < S::kCG; ++cg)
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int r = 0; r < kRegs; ++r) acc[cg][j][r] = 0.0f;
+
+  struct Regs {
+    f32x4 x;
+    f32x4 y[4][S::kCG];
+  };
+  auto mma = [&](const Regs& o) {
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int cg = 0; cg < S::kCG; ++cg)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[cg][j] = A::mma(o.x[t], o.y[t][cg][j], acc[cg][j]);
+  };
+  // a group whose columns or k may lie outside the matrix: rows of W past D
+  // read as 0
+  auto load_any = [&](int g, Regs& o) {
+    o.x = *reinterpret_cast<const f32x4*>(act + (size_t)g * S::kG * R);
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const int k = g * S::kG + S::kQ * t + q;
+      const float* p = a.w + (size_t)min(k, D - 1) * a.ldw;
+#pragma unroll
+      for (int cg = 0; cg < S::kCG; ++cg)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float y = p[min(v0 + 4 * c + 4 * R * cg + e, V - 1)];
+          o.y[t][cg][e] = k < D ? y : 0.0f;
+        }
+    }
+  };
+
+  const int full = D / S::kG;  // groups whose k all lie inside D: wave w takes w, w + 8, ...
+  if constexpr (ANY) {
+    for (int g = w; g * S::kG < D; g += kWaves) {
+      Regs o;
+      load_any(g, o);
+      mma(o);
+    }
+  } else {
+    if (full * S::kG < D && w == full % kWaves) {
+      Regs o;
+      load_any(full, o);
+      mma(o);
+    }
+    const int voff = (int)(q * a.ldw + 4 * c) * 4, row = (int)(S::kQ * a.ldw) * 4;
+    auto load = [&](int g, Regs& o) {
+      const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+          const_cast<float*>(a.w + (size_t)g * S::kG * a.ldw + v0), (short)0, 0x7fffffff, 0x00020000);
+      o.x = *reinterpret_cast<const f32x4*>(act + (size_t)g * S::kG * R);
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int cg = 0; cg < S::kCG; ++cg)
+          o.y[t][cg] = __builtin_bit_cast(
+              f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, voff + 16 * R * cg, row * t, 0));
+    };
+    // the next group's loads are in flight while this one is multiplied
+    Regs r0, r1;
+    if (w < full) load(w, r0);
+    for (int g = w; g < full; g += 2 * kWaves) {
+      if (g + kWaves < full) load(g + kWaves, r1);
+      __builtin_amdgcn_sched_barrier(0);
+      mma(r0);
+      __builtin_amdgcn_sched_barrier(0);
+      if (g + kWaves < full) {
+        if (g + 2 * kWaves < full) load(g + 2 * kWaves, r0);
+        __builtin_amdgcn_sched_barrier(0);
+        mma(r1);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+  }
+
+  // the waves' sums, in the order ((0+4)+(2+6)) + ((1+5)+(3+7)); each lane's
+  // four column tiles travel as one 16-byte value
+#pragma unroll
+  for (int half = kWaves / 2; half >= 1; half >>= 1) {
+    if (w >= half && w < 2 * half) {
+#pragma unroll
+      for (int cg = 0; cg < S::kCG; ++cg)
+#pragma unroll
+        for (int r = 0; r < kRegs; ++r)
+          sm[w - half][cg * kRegs + r][l] = f32x4{acc[cg][0][r], acc[cg][1][r], acc[cg][2][r], acc[cg][3][r]};
+    }
+    wg_barrier();
+    if (w < half) {
+#pragma unroll
+      for (int cg = 0; cg < S::kCG; ++cg)
+#pragma unroll
+        for (int r = 0; r < kRegs; ++r) {
+          const f32x4 o = sm[w][cg * kRegs + r][l];
+#pragma unroll
+          for (int j = 0; j < 4; ++j) acc[cg][j][r] += o[j];
+        }
+    }
+    wg_barrier();
+  }
+  if (w != 0) return;
+#pragma unroll
+  for (int cg = 0; cg < S::kCG; ++cg)
+#pragma unroll
+    for (int r = 0; r < kRegs; ++r) {
+      const int n = A::row(r, l);
+      const int v = v0 + 4 * c + 4 * R * cg;
+      if (n >= a.N) continue;
+      float* o = a.out + (size_t)n * a.ldo + v;
+      const f32x4 y{acc[cg][0][r], acc[cg][1][r], acc[cg][2][r], acc[cg][3][r]};
+      if constexpr (ANY) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          if (v + j < V) o[j] = y[j];
+      } else {
+        *reinterpret_cast<f32x4u*>(o) = y;
+      }
+    }
+}
+
+template <int R>
+hipError_t launch_head_skinny(const HeadArgs& a, hipStream_t s) {
+  hipLaunchKernelGGL(k_head_prep<R>, dim3(a.N), dim3(kThreads), 0, s, a);
+  const dim3 grid((unsigned)((a.V + kSkinnyCols - 1) / kSkinnyCols));
+  if (a.V < kSkinnyCols || a.ldw > (1 << 24)) hipLaunchKernelGGL((k_head_skinny<R, true>), grid, dim3(kThreads), 0, s, a);
+  else hipLaunchKernelGGL((k_head_skinny<R, false>), grid, dim3(kThreads), 0, s, a);
+  return hipGetLastError();
+}
+
 size_t head_ws_bytes(int N, int D) {
   return ((size_t)head_kpad(D) * head_npad(N) + (size_t)N) * sizeof(float) + 256;
 }
 
 hipError_t launch_head(HeadArgs a, hipStream_t s) {
+  // up to 32 rows the product is bound by the one read of W, not by the
+  // matrix cores (at 157 TFLOP/s 32 rows take half of W's time in HBM)
+  if (a.N <= 16) return launch_head_skinny<16>(a, s);
+  if (a.N <= 32) return launch_head_skinny<32>(a, s);
   // workspace: act [Dp][lda] (k-major), then rinv [N]
   a.lda = head_npad(a.N);
   a.rinv = a.act + (size_t)head_kpad(a.D) * a.lda;

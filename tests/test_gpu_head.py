@@ -50,6 +50,35 @@ def test_head_matches_oracle(N, D, V):
     np.testing.assert_allclose(got, ref, rtol=1e-4, atol=1e-4)
 
 
+@pytest.mark.parametrize("N", [1, 16, 17, 32])          # the row counts at which the few-rows kernels change
+@pytest.mark.parametrize("D,V", [
+    (8, 127),    # one column short of a workgroup; k ends in a ragged group (16 rows) or a whole one (32)
+    (128, 128),  # one workgroup, whole groups, one k group per wave at 16 rows
+    (129, 129),  # the last workgroup's columns overlap the first's; one k past the whole groups
+    (1000, 333),
+])
+def test_few_rows(N, D, V):
+    """The few-rows kernels on W, h and out rows of odd strides (no 16-byte
+    alignment anywhere), nothing written outside out."""
+    import torch
+
+    print(f"[head] few rows N={N} D={D} V={V}", flush=True)
+    h, norm, W = _case(N + D, N, D, V)
+    wb = torch.full((D, V + 3), float("nan"), device="cuda")
+    wb[:, 1:V + 1] = torch.from_numpy(W).cuda()
+    hb = torch.full((N, D + 1), float("nan"), device="cuda")
+    hb[:, :D] = torch.from_numpy(h).cuda()
+    ob = torch.full((N + 1, V + 5), 7.0, device="cuda")
+    torch.cuda.synchronize()
+    H.rms_norm_lm_head(hb[:, :D], torch.from_numpy(norm).cuda(), wb[:, 1:V + 1], 1e-5, out=ob[:N, :V])
+    torch.cuda.synchronize()
+    got = ob.cpu().numpy()
+    bound = oracle.head_error_bound(h, norm, W, 1e-5)
+    err = np.abs(got[:N, :V].astype(np.float64) - oracle.lm_head_logits(h, norm, W, 1e-5))
+    assert np.all(err <= TOL * bound + 1e-30), float(np.max(err / (bound + 1e-30)))
+    assert np.all(got[N:] == 7.0) and np.all(got[:, V:] == 7.0)
+
+
 def test_tiny_rows_and_eps():
     """Rows of norm ~1e-3 (eps visible), an all-zero row (r = 1/sqrt(eps))."""
     h, norm, W = _case(3, 6, 96, 257, scale=1e-3)
