@@ -757,8 +757,9 @@ def bench_head(steps: int = 20, warmup: int = 3, N: int = 256, D: int = 4096, V:
     """The logits producer at the sampler's headline shape: final RMSNorm and
     lm_head (256 rows, model width 4096, 128 256-token vocabulary, float32
     weights resident in HBM, random-init) writing the logits the sampler
-    reads.  Reports launches/s of the pair and the product's float32 matrix
-    rate against the 157.3 TFLOP/s fp32 MFMA peak."""
+    reads.  Reports launches/s of the pair and the product's rate in float32
+    operations; against the 157.3 TFLOP/s fp32 MFMA peak it can exceed 1, as
+    each float32 product is six exact bf16 products."""
     import torch
 
     from pagellm_amd import _native

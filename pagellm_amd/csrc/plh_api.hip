@@ -592,7 +592,7 @@ int plh_rmsnorm_lm_head(plh_ctx* c, const float* h, int64_t ldh, int N, int D, c
   if (!(eps >= 0.0) || !std::isfinite(eps)) return fail(c, PLH_ERR_INVALID_ARG, "eps must be finite and >= 0%s");
   int rc = use_device(c);
   if (rc != PLH_OK) return rc;
-  rc = reserve_ws(c, plh::head_ws_bytes(N, D));
+  rc = reserve_ws(c, plh::head_ws_bytes(N, D, V, ldw, c->num_cu));
   if (rc != PLH_OK) return rc;
   plh::HeadArgs a{};
   a.h = h;
@@ -603,11 +603,11 @@ int plh_rmsnorm_lm_head(plh_ctx* c, const float* h, int64_t ldh, int N, int D, c
   a.ldw = ldw;
   a.out = out;
   a.ldo = ldo;
-  a.act = static_cast<float*>(c->ws);
+  a.act = c->ws;
   a.N = N;
   a.D = D;
   a.V = V;
-  const hipError_t e = plh::launch_head(a, c->stream);
+  const hipError_t e = plh::launch_head(a, c->num_cu, c->stream);
   if (e != hipSuccess) return hip_fail(c, e, "plh_rmsnorm_lm_head launch");
   c->ws_stream = c->stream;
   c->ws_open = true;

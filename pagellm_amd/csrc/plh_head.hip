@@ -3,46 +3,28 @@
 // (src/pagellm/model/transformer.py:79-82, :271), in float32 as the
 // reference computes it, written straight into the sampler's logits buffer.
 //
-//   k_head_rms      one workgroup per row: r = 1 / sqrt(mean(h * h) + eps)
-//                   in float32 (the squares summed in float64 and rounded
-//                   once);
-//   k_head_act      act = (h * r) * norm, stored k-major and zero-padded to
-//                   whole tiles (32 in k, 256 in n);
-//   k_head_prep,    the same for at most 32 rows (see "few rows" below);
-//   k_head_skinny
-//   k_head_gemm     out = act @ W on the fp32 matrix cores
-//                   (v_mfma_f32_32x32x2_f32, products and sums in float32).
-//                   A workgroup of 8 waves (two per SIMD) owns a 256-row x
-//                   256-column tile of out; each wave a 64 x 128 block,
-//                   2 x 4 MFMA tiles held in 128 accumulator registers.
-//                   Both operands are k-major in LDS (each half-wave reads
-//                   32 consecutive floats per MFMA operand); k streams
-//                   through LDS 32 at a time, double-buffered: the next
-//                   stage is copied from HBM straight into LDS
-//                   (global_load_lds_dwordx4) while the matrix cores work on
-//                   the current one, and operand reads run two k steps ahead
-//                   of the MFMAs.
+// Two launches: a prep kernel (one workgroup per row: RMSNorm with numpy's
+// float32 steps, and act = (h * r) * norm in the layout the product reads),
+// then the product:
+//
+//   k_head_skinny   at most 32 rows: one read of W, fp32 matrix cores
+//   k_head_split    more rows: float32 products on the bf16 matrix cores,
+//                   each operand split exactly into three bf16 parts
 #include "plh_device.h"
 #include "plh_kernels.h"
+
+#include <algorithm>
+#include <cmath>
 
 namespace plh {
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-constexpr int kHeadRows = 256;             // rows of out per workgroup
-constexpr int kHeadCols = 256;             // vocabulary columns per workgroup
-constexpr int kHeadK = 32;                 // k per LDS stage
-constexpr int kTileStride = 256 + 32;      // LDS row pitch of both tiles (floats)
-
-__host__ __device__ constexpr int head_kpad(int D) { return (D + kHeadK - 1) / kHeadK * kHeadK; }
-__host__ __device__ constexpr int head_npad(int N) { return (N + kHeadRows - 1) / kHeadRows * kHeadRows; }
-
-// r_n = 1 / sqrt(mean(h[n] * h[n]) + eps), one workgroup per row.
-__global__ __launch_bounds__(kThreads) void k_head_rms(HeadArgs a) {
+// r = 1 / sqrt(mean(x * x) + eps) of a row of h, the same bits in every thread
+// of the workgroup.
+__device__ __forceinline__ float row_rinv(const HeadArgs& a, const float* x) {
   __shared__ double red[kWaves];
-  const int n = blockIdx.x;
-  const float* x = a.h + (size_t)n * a.ldh;
   double s = 0.0;
   for (int d = threadIdx.x; d < a.D; d += kThreads) {
     const float v = x[d];
@@ -51,224 +33,19 @@ __global__ __launch_bounds__(kThreads) void k_head_rms(HeadArgs a) {
   s = block_sum(s, red);
   // np.mean in float32, + eps as a float32 (a Python float is a weak
   // scalar), float32 sqrt and reciprocal (transformer.py:81)
-  if (threadIdx.x == 0) {
-    const float mean = (float)s / (float)a.D;
-    a.rinv[n] = 1.0f / sqrtf(mean + a.eps);
-  }
+  return 1.0f / sqrtf((float)s / (float)a.D + a.eps);
 }
 
-// act[d][n] = (h[n][d] * r_n) * norm[d] (transformer.py:82), stored k-major
-// ([Dp][lda], lda = N rounded up to the row tile) and zero outside
-// d < D, n < N: a 32 (d) x 64 (n) block per workgroup, transposed through LDS
-// so that both the reads of h and the writes of act are 16-byte and
-// contiguous.
-__global__ __launch_bounds__(kThreads) void k_head_act(HeadArgs a) {
-  __shared__ float t[64][32 + 1];
-  const int d0 = blockIdx.x * 32, n0 = blockIdx.y * 64;
-  const int tid = threadIdx.x;
-  {
-    const int nl = tid >> 3, dl = (tid & 7) * 4;  // 64 rows x 8 groups of 4
-    const int n = n0 + nl;
-    float v[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-    if (n < a.N) {
-      const float r = a.rinv[n];
-      const float* x = a.h + (size_t)n * a.ldh;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int d = d0 + dl + e;
-        if (d < a.D) v[e] = (x[d] * r) * a.norm[d];
-      }
-    }
-#pragma unroll
-    for (int e = 0; e < 4; ++e) t[nl][dl + e] = v[e];
-  }
-  wg_barrier();
-  {
-    const int dl = tid >> 4, nl = (tid & 15) * 4;  // 32 rows x 16 groups of 4
-    f32x4 v;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) v[e] = t[nl + e][dl];
-    *reinterpret_cast<f32x4*>(a.act + (size_t)(d0 + dl) * a.lda + n0 + nl) = v;
-  }
-}
-
-// 16-byte aligned, so that the stage stores are single ds_write_b128s
-struct __attribute__((aligned(16))) HeadSmem {
-  float a[2][kHeadK * kTileStride];  // act stage, [k][n]
-  float b[2][kHeadK * kTileStride];  // W stage, [k][v]
+// Where a product kernel's sums go: out, or with several slices of k
+// (gridDim.z) the slice's own [N, V] partial sums, which k_head_sum adds up.
+struct HeadOut {
+  float* p;
+  size_t ld;
 };
 
-// Wave layout: each wave owns kMT x 4 MFMA tiles (kMT * 32 rows x 128
-// columns) of the workgroup's 256 x 256 tile.  kMT = 2: 8 waves, two per
-// SIMD, 128 accumulators each; kMT = 4: 4 waves, one per SIMD, 256.
-constexpr int kMT = 2;
-constexpr int kWavesN = kHeadRows / (32 * kMT);
-constexpr int kGemmWaves = kWavesN * 2;
-constexpr int kGemmThreads = 64 * kGemmWaves;
-constexpr int kStageRows = kGemmThreads / 64;   // stage rows one pass of the workgroup moves
-constexpr int kStagePasses = kHeadK / kStageRows;
-// The next stage goes to LDS one pass (two ds_write_b128) per k step,
-// after steps kStoreStep .. kStoreStep + kStagePasses - 1, so that LDS
-// writes never arrive as a burst in front of the operand reads.
-constexpr int kStoreStep = 1;
-constexpr int kAhead = 2;                        // k steps the operand reads run ahead
-static_assert(kStoreStep + kStagePasses <= kHeadK / 2, "stage stores must end inside the k loop");
-
-// One workgroup tile.  VEC: every W row segment of the tile is inside the
-// matrix and 16-byte aligned (all tiles but a ragged last one); the two
-// forms are separate code so that no branch joins inside the k loop.
-// DMA (full tiles whose k stages all lie inside D): the stages go from HBM
-// straight into LDS (global_load_lds_dwordx4: each wave's load fills one
-// contiguous 1 KB LDS row, lane l at 16 l), with no registers or LDS
-// stores on the way; the wave waits for its copies before the barrier that
-// ends the stage.
-template <bool VEC, bool DMA>
-__device__ __forceinline__ void head_tile(const HeadArgs& a, HeadSmem& sm) {
-  static_assert(!DMA || VEC, "the DMA form needs whole, aligned rows");
-  const int N = a.N, D = a.D, V = a.V;
-  const int v0 = blockIdx.x * kHeadCols, n0 = blockIdx.y * kHeadRows;
-  const int tid = threadIdx.x, l = lane(), w = wave();
-  const int wn = w % kWavesN, wv = w / kWavesN;  // this wave's block of the tile
-
-  // global -> register staging, the same map for both tiles: stage row
-  // (tid / 64) + kStageRows j, 4 columns from (tid % 64) * 4, so that each wave moves
-  // one contiguous 1 KB row per load and per LDS store.  act is padded to
-  // whole tiles; W rows past D are read clamped and zeroed at the store.
-  const int sr = tid >> 6, sc = (tid & 63) * 4;
-  const float* ag = a.act + (size_t)sr * a.lda + n0 + sc;
-  // The loads only fill registers; what falls outside the matrix is zeroed
-  // when the registers go to LDS, so that no wait for the loads precedes
-  // the current stage's MFMAs.
-  f32x4 pa[kStagePasses], pb[kStagePasses];
-  auto load = [&](int kb) {
-    const int k0 = kb * kHeadK;
-#pragma unroll
-    for (int j = 0; j < kStagePasses; ++j)
-      pa[j] = *reinterpret_cast<const f32x4*>(ag + (size_t)(k0 + kStageRows * j) * a.lda);
-#pragma unroll
-    for (int j = 0; j < kStagePasses; ++j) {
-      const float* bg = a.w + (size_t)min(k0 + sr + kStageRows * j, D - 1) * a.ldw;
-      if constexpr (VEC) {
-        pb[j] = *reinterpret_cast<const f32x4*>(bg + v0 + sc);
-      } else {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) pb[j][e] = bg[min(v0 + sc + e, V - 1)];
-      }
-    }
-  };
-  auto store = [&](int kb, int buf, int j) {
-    {
-      const int r = sr + kStageRows * j;
-      *reinterpret_cast<f32x4*>(sm.a[buf] + r * kTileStride + sc) = pa[j];
-      const bool kin = kb * kHeadK + r < D;
-      f32x4 v = pb[j];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] = (kin && v0 + sc + e < V) ? v[e] : 0.0f;
-      *reinterpret_cast<f32x4*>(sm.b[buf] + r * kTileStride + sc) = v;
-    }
-  };
-
-  f32x16 acc[kMT][4];
-#pragma unroll
-  for (int mt = 0; mt < kMT; ++mt)
-#pragma unroll
-    for (int nt = 0; nt < 4; ++nt)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[mt][nt][r] = 0.0f;
-
-  // the DMA form: stage kb into LDS buffer buf (the LDS row of each copy is
-  // the same for the whole wave, as the instruction requires)
-  auto dma = [&](int kb, int buf) {
-    const int k0 = kb * kHeadK;
-#pragma unroll
-    for (int j = 0; j < kStagePasses; ++j) {
-      const int r = sr + kStageRows * j;
-      __builtin_amdgcn_global_load_lds(ag + (size_t)(k0 + kStageRows * j) * a.lda, sm.a[buf] + r * kTileStride, 16,
-                                       0, 0);
-      __builtin_amdgcn_global_load_lds(a.w + (size_t)(k0 + r) * a.ldw + v0 + sc, sm.b[buf] + r * kTileStride, 16, 0,
-                                       0);
-    }
-  };
-  auto dma_wait = [] { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); };
-
-  const int nkb = head_kpad(D) / kHeadK;
-  if constexpr (DMA) {
-    dma(0, 0);
-    dma_wait();
-  } else {
-    load(0);
-#pragma unroll
-    for (int j = 0; j < kStagePasses; ++j) store(0, 0, j);
-  }
-  wg_barrier();
-  for (int kb = 0; kb < nkb; ++kb) {
-    const int cur = kb & 1;
-    if constexpr (DMA) {
-      if (kb + 1 < nkb) dma(kb + 1, cur ^ 1);  // the other buffer's last reads were before the barrier
-    } else {
-      if (kb + 1 < nkb) load(kb + 1);
-    }
-    // operands of v_mfma_f32_32x32x2_f32 at k step t: lane l holds
-    // A[row l%32][k 2t + l/32] and B[k 2t + l/32][column l%32]; both tiles
-    // are k-major, so each half-wave reads 32 consecutive floats
-    const float* as = sm.a[cur] + (l >> 5) * kTileStride + wn * 32 * kMT + (l & 31);
-    const float* bs = sm.b[cur] + (l >> 5) * kTileStride + wv * 128 + (l & 31);
-    // the operands of step t + kAhead are read from LDS while step t's
-    // MFMAs run
-    float fa[kAhead + 1][kMT], fb[kAhead + 1][4];
-    auto frags = [&](int t, int slot) {
-#pragma unroll
-      for (int i = 0; i < kMT; ++i) fa[slot][i] = as[2 * t * kTileStride + 32 * i];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) fb[slot][i] = bs[2 * t * kTileStride + 32 * i];
-    };
-#pragma unroll
-    for (int t = 0; t < kAhead; ++t) frags(t, t);
-#pragma unroll
-    for (int t = 0; t < kHeadK / 2; ++t) {
-      const int sl = t % (kAhead + 1);
-      if (t + kAhead < kHeadK / 2) frags(t + kAhead, (t + kAhead) % (kAhead + 1));
-      __builtin_amdgcn_sched_barrier(0);  // keep the reads ahead of the MFMAs
-#pragma unroll
-      for (int nt = 0; nt < 4; ++nt)
-#pragma unroll
-        for (int mt = 0; mt < kMT; ++mt)
-          acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[sl][mt], fb[sl][nt], acc[mt][nt], 0, 0, 0);
-      __builtin_amdgcn_sched_barrier(0);
-      // the next stage goes to the other LDS buffer (its last reads were
-      // before the previous barrier)
-      if constexpr (!DMA) {
-        if (t >= kStoreStep && t < kStoreStep + kStagePasses && kb + 1 < nkb)
-          store(kb + 1, cur ^ 1, t - kStoreStep);
-      }
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    if constexpr (DMA) dma_wait();
-    wg_barrier();
-  }
-
-  // accumulator r of lane l holds row 8*(r/4) + 4*(l/32) + r%4, column l%32
-#pragma unroll
-  for (int mt = 0; mt < kMT; ++mt)
-#pragma unroll
-    for (int nt = 0; nt < 4; ++nt) {
-      const int v = v0 + wv * 128 + nt * 32 + (l & 31);
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int n = n0 + wn * 32 * kMT + mt * 32 + 8 * (r >> 2) + 4 * (l >> 5) + (r & 3);
-        if (n < N && v < V) a.out[(size_t)n * a.ldo + v] = acc[mt][nt][r];
-      }
-    }
-}
-
-__global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(kGemmWaves / 4, kGemmWaves / 4))) void
-k_head_gemm(HeadArgs a) {
-  __shared__ HeadSmem sm;
-  const int v0 = blockIdx.x * kHeadCols;
-  const bool vec = v0 + kHeadCols <= a.V && (a.ldw & 3) == 0 && (reinterpret_cast<uintptr_t>(a.w) & 15) == 0;
-  if (vec && a.D % kHeadK == 0) head_tile<true, true>(a, sm);
-  else if (vec) head_tile<true, false>(a, sm);
-  else head_tile<false, false>(a, sm);
+__device__ __forceinline__ HeadOut head_out(const HeadArgs& a) {
+  if (gridDim.z == 1) return HeadOut{a.out, (size_t)a.ldo};
+  return HeadOut{a.part + (size_t)blockIdx.z * a.N * a.V, (size_t)a.V};
 }
 
 // ------------------------------------------------------------- few rows
@@ -310,21 +87,14 @@ __host__ __device__ constexpr int skinny_groups(int D, int R) { return (D + 256 
 template <int R>
 __global__ __launch_bounds__(kThreads) void k_head_prep(HeadArgs a) {
   using S = Skinny<R>;
-  __shared__ double red[kWaves];
   const int n = blockIdx.x, D = a.D;
   const float* x = a.h + (size_t)n * a.ldh;
-  double s = 0.0;
-  for (int d = threadIdx.x; d < D; d += kThreads) {
-    const float v = x[d];
-    s += (double)(v * v);  // the float32 square, as numpy forms x * x
-  }
-  s = block_sum(s, red);
-  // as in k_head_rms, by every thread alike
-  const float r = 1.0f / sqrtf((float)s / (float)D + a.eps);
-  const int Dp = skinny_groups(D, R) * S::kG;
-  for (int d = threadIdx.x; d < Dp; d += kThreads) {
+  const float r = row_rinv(a, x);
+  const int groups = skinny_groups(D, R);
+  float* o = static_cast<float*>(a.act) + (size_t)(n / R) * groups * S::kG * R;
+  for (int d = threadIdx.x; d < groups * S::kG; d += kThreads) {
     const int g = d / S::kG, e = d % S::kG;
-    a.act[((size_t)(g * S::kQ + e % S::kQ) * R + n) * 4 + e / S::kQ] = d < D ? (x[d] * r) * a.norm[d] : 0.0f;
+    o[((size_t)(g * S::kQ + e % S::kQ) * R + n % R) * 4 + e / S::kQ] = d < D ? (x[d] * r) * a.norm[d] : 0.0f;
   }
 }
 
@@ -365,7 +135,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
   const int D = a.D, V = a.V, l = lane(), w = uniform(wave());
   const int v0 = ANY ? (int)blockIdx.x * kSkinnyCols : min((int)blockIdx.x * kSkinnyCols, V - kSkinnyCols);
   const int c = l % R, q = l / R;
-  const float* act = a.act + (size_t)(q * R + c) * 4;
+  const int n0 = blockIdx.y * R;
+  const float* act =
+      static_cast<const float*>(a.act) + (size_t)blockIdx.y * skinny_groups(D, R) * S::kG * R + (size_t)(q * R + c) * 4;
 
   typename A::T acc[S::kCG][4];
 #pragma unroll
@@ -405,15 +177,17 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
     }
   };
 
-  const int full = D / S::kG;  // groups whose k all lie inside D: wave w takes w, w + 8, ...
+  // groups whose k all lie inside D; with several slices of k (blockIdx.z)
+  // wave w of slice z takes w + 8 z, w + 8 (z + slices), ...
+  const int full = D / S::kG, step = kWaves * (int)gridDim.z, g0 = w + kWaves * (int)blockIdx.z;
   if constexpr (ANY) {
-    for (int g = w; g * S::kG < D; g += kWaves) {
+    for (int g = g0; g * S::kG < D; g += step) {
       Regs o;
       load_any(g, o);
       mma(o);
     }
   } else {
-    if (full * S::kG < D && w == full % kWaves) {
+    if (full * S::kG < D && g0 == full % step) {
       Regs o;
       load_any(full, o);
       mma(o);
@@ -432,14 +206,14 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
     };
     // the next group's loads are in flight while this one is multiplied
     Regs r0, r1;
-    if (w < full) load(w, r0);
-    for (int g = w; g < full; g += 2 * kWaves) {
-      if (g + kWaves < full) load(g + kWaves, r1);
+    if (g0 < full) load(g0, r0);
+    for (int g = g0; g < full; g += 2 * step) {
+      if (g + step < full) load(g + step, r1);
       __builtin_amdgcn_sched_barrier(0);
       mma(r0);
       __builtin_amdgcn_sched_barrier(0);
-      if (g + kWaves < full) {
-        if (g + 2 * kWaves < full) load(g + 2 * kWaves, r0);
+      if (g + step < full) {
+        if (g + 2 * step < full) load(g + 2 * step, r0);
         __builtin_amdgcn_sched_barrier(0);
         mma(r1);
         __builtin_amdgcn_sched_barrier(0);
@@ -472,14 +246,15 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
     wg_barrier();
   }
   if (w != 0) return;
+  const HeadOut to = head_out(a);
 #pragma unroll
   for (int cg = 0; cg < S::kCG; ++cg)
 #pragma unroll
     for (int r = 0; r < kRegs; ++r) {
-      const int n = A::row(r, l);
+      const int n = n0 + A::row(r, l);
       const int v = v0 + 4 * c + 4 * R * cg;
       if (n >= a.N) continue;
-      float* o = a.out + (size_t)n * a.ldo + v;
+      float* o = to.p + (size_t)n * to.ld + v;
       const f32x4 y{acc[cg][0][r], acc[cg][1][r], acc[cg][2][r], acc[cg][3][r]};
       if constexpr (ANY) {
 #pragma unroll
@@ -491,32 +266,390 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
     }
 }
 
+// ------------------------------------------------------------ many rows
+//
+// float32 products on the bf16 matrix cores.  A float32 x is exactly
+// hi + mid + lo, three bf16 values (its 24 significant bits, 8 at a time), so
+//   a * w = ah*wh + (ah*wm + am*wh) + (ah*wl + am*wm + al*wh) + rest,
+// with |rest| <= 2^-22 |a w| (three products of 2^-8 * 2^-16 and below), each
+// product exact and summed in float32 by v_mfma_f32_32x32x16_bf16.  Six bf16
+// products cost 6/16 of one on the fp32 matrix cores (2.5 PFLOP/s against 157
+// TFLOP/s), and a sum over k is rounded 6 times per 16 k instead of 8.
+// Against float64 the result is no further off than the fp32 matrix product
+// (2-norm, N(0, 1) rows, 0.02 N(0, 1) weights): 1.02e-6 against 1.1e-6 at
+// D = 4096, 4.9e-7 against 5.6e-7 at 1000, less with several slices of k.
+//
+// k_head_split<BM>: a BM-row x 256-column tile per workgroup, 8 waves of 64
+// rows x (BM / 2) columns (at least 32), k in stages of 16.  act comes split
+// from the prep kernel.  A thread holds one column's 8 k values of W (read
+// coalesced over the lanes, so rows of any alignment are read alike), splits
+// them and stores the three parts for the whole workgroup in LDS,
+// double-buffered; LDS is read and written 16 bytes a lane, consecutive lanes
+// consecutive pieces.  Both operands' loads run kPF stages ahead in registers.
+// They are issued together: loads return in order, and an operand loaded one
+// stage ahead on its own made every stage wait for the other's newest loads
+// (4096 x 128 256: 64 rows 690 us, 256 rows 1 420 us).  The stage loop has no
+// branch and no predicated load for the same reason: at a join the loads'
+// registers were copied, which waits for them.
+// Inputs that the split cannot carry (infinities, float32 overflow on the
+// way, results so small that bf16 parts underflow) show up in the result;
+// the wave then forms its tile again on the fp32 matrix cores.
+//
+// Against the fp32 matrix product in 256-row tiles, 4096 x 128 256: 256 rows
+// 2 020 -> 1 230 us (1.31 PFLOP/s of bf16 products, the rate of a large bf16
+// matrix product here), 128 rows 2 000 -> 740 us, 64 rows 2 000 -> 590 us, bound
+// by W's way through a CU; 45 x 1000 x 50 257: 293 -> 61 us.
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+constexpr int kSplitCols = 256;  // columns per workgroup
+constexpr int kSplitK = 16;      // k per stage: one MFMA step
+constexpr int kSplitMaxLdw = 1 << 24;  // a stage's rows of W lie within 2^30 bytes
+
+__host__ __device__ constexpr int split_stages(int D) { return (D + kSplitK - 1) / kSplitK; }
+
+struct Split8 {
+  u32x4 part[3];  // hi, mid, lo: 8 bf16 each
+};
+
+// x = hi + mid + lo by truncation: each remainder is exact.
+__device__ __forceinline__ Split8 split8(const float (&x)[8]) {
+  Split8 s;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    float a = x[2 * i], b = x[2 * i + 1];
+#pragma unroll
+    for (int p = 0; p < 3; ++p) {
+      const uint32_t ua = __float_as_uint(a), ub = __float_as_uint(b);
+      s.part[p][i] = __builtin_amdgcn_perm(ub, ua, 0x07060302u);  // the upper halves of b and a
+      if (p < 2) {
+        a -= __uint_as_float(ua & 0xffff0000u);
+        b -= __uint_as_float(ub & 0xffff0000u);
+      }
+    }
+  }
+  return s;
+}
+
+// act for k_head_split: part p, k group kg (8 k), row n at
+// ((p * groups + kg) * lda + n) * 8; zero for k >= D (rows N .. lda-1 are not
+// written: an accumulator row depends on its own act row only).
+__global__ __launch_bounds__(kThreads) void k_head_prep_split(HeadArgs a) {
+  const int n = blockIdx.x, D = a.D;
+  const float* x = a.h + (size_t)n * a.ldh;
+  const float r = row_rinv(a, x);
+  const int groups = 2 * split_stages(D);
+  u32x4* o = static_cast<u32x4*>(a.act);
+  for (int kg = threadIdx.x; kg < groups; kg += kThreads) {
+    float v[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const int d = 8 * kg + e;
+      v[e] = d < D ? (x[d] * r) * a.norm[d] : 0.0f;
+    }
+    const Split8 s = split8(v);
+#pragma unroll
+    for (int p = 0; p < 3; ++p) o[((size_t)p * groups + kg) * a.lda + n] = s.part[p];
+  }
+}
+
+// A sum that the bf16 parts may not carry: not finite, or below 2^-80 without
+// being 0.
+__device__ __forceinline__ bool split_suspect(float x) {
+  const float y = fabsf(x);
+  return !(y <= 3.4028234663852886e38f) || (y < 8.2718061255302767e-25f && y > 0.0f);
+}
+
+// act[n][k] in float32, from its parts (exact; a non-finite value is all in
+// its first part, a NaN in the first two)
+__device__ __forceinline__ float split_act(const HeadArgs& a, int n, int k) {
+  const uint16_t* act = static_cast<const uint16_t*>(a.act);
+  const int groups = 2 * split_stages(a.D);
+  float part[3];
+#pragma unroll
+  for (int p = 0; p < 3; ++p)
+    part[p] = __uint_as_float((uint32_t)act[(((size_t)p * groups + (k >> 3)) * a.lda + n) * 8 + (k & 7)] << 16);
+  return part[1] != part[1] ? (part[0] == part[0] ? part[0] : part[1]) : part[0] + (part[1] + part[2]);
+}
+
+// One 32 x 32 tile of out, rows n.. and columns v.., on the fp32 matrix cores.
+__device__ __forceinline__ f32x16 head_tile_f32(const HeadArgs& a, int n, int v) {
+  const int l = lane(), D = a.D;
+  const int row = n + (l & 31), col = min(v + (l & 31), a.V - 1);
+  f32x16 acc;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
+#pragma unroll 8
+  for (int k0 = 0; k0 < D; k0 += 2) {
+    const int k = k0 + (l >> 5), kc = min(k, D - 1);
+    const float x = split_act(a, row, kc);
+    const float y = a.w[(size_t)kc * a.ldw + col];
+    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(k < D ? x : 0.0f, k < D ? y : 0.0f, acc, 0, 0, 0);
+  }
+  return acc;
+}
+
+template <int BM>
+struct SplitGeo {
+  static constexpr int kWR = BM / 64;                         // waves along the rows
+  static constexpr int kNT = kSplitCols / 32 * kWR / kWaves;  // 32-column tiles per wave
+  static constexpr int kA = (6 * BM + kThreads - 1) / kThreads;  // 16-byte pieces of act per thread and stage
+  static constexpr int kPF = BM <= 128 ? 4 : 2;               // stages in registers
+  static constexpr int kEu = BM == 64 ? 4 : 2;                // waves per SIMD
+};
+
+template <int BM>
+struct SplitSmem {
+  u32x4 a[2][SplitGeo<BM>::kA * kThreads];  // [buffer][(part * 2 + k group) * BM + row], and a thread's unused pieces
+  u32x4 b[2][3][2][kSplitCols];    // [buffer][part][k group][column]
+};
+
+template <int BM>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(SplitGeo<BM>::kEu, SplitGeo<BM>::kEu))) void
+k_head_split(HeadArgs a) {
+  using G = SplitGeo<BM>;
+  constexpr int kNT = G::kNT, kPF = G::kPF;
+  __shared__ SplitSmem<BM> sm;
+  const int D = a.D, V = a.V, l = lane(), w = uniform(wave());
+  // the row tiles of one column tile run side by side, so that all but the
+  // first find W in the caches
+  const int rt = (int)a.lda / BM;
+  const int v0 = (int)(blockIdx.x / rt) * kSplitCols, n0 = (int)(blockIdx.x % rt) * BM;
+  const int wr = w % G::kWR, wc = w / G::kWR;
+  // this slice's stages, a multiple of kPF (the last slice's stages past nk
+  // multiply W by 0)
+  const int nk = split_stages(D), groups = 2 * nk, units = (nk + kPF - 1) / kPF;
+  const int sb = (int)((int64_t)units * blockIdx.z / gridDim.z) * kPF;
+  const int se = (int)((int64_t)units * (blockIdx.z + 1) / gridDim.z) * kPF;
+
+  // W: this thread's column and k group (uniform over the wave); act: 16-byte
+  // pieces tid, tid + 512, ... of the stage's 6 BM
+  const int col = (int)threadIdx.x & (kSplitCols - 1), kg = w >> 2;
+  const int pitch = (int)a.ldw * 4;
+  float wreg[kPF][8];
+  u32x4 areg[kPF][G::kA];
+  auto load = [&](int s, float (&o)[8], u32x4 (&x)[G::kA]) {
+    const int rows = min(D - s * kSplitK, kSplitK);  // rows past D, and stages past the slice's, read as 0
+    const int bytes = s < se && rows > 0 ? (rows - 1) * pitch + (V - v0) * 4 : 0;
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<float*>(a.w + (size_t)s * kSplitK * a.ldw + v0), (short)0, bytes, 0x00020000);
+    const u32x4* ap = static_cast<const u32x4*>(a.act) + (size_t)(2 * min(s, nk - 1)) * a.lda + n0;
+#pragma unroll
+    for (int i = 0; i < G::kA; ++i) {
+      const int q = min((int)threadIdx.x + kThreads * i, 6 * BM - 1);
+      x[i] = ap[((size_t)(q / (2 * BM)) * groups + (q / BM) % 2) * a.lda + q % BM];
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      o[j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, col * 4, (kg * 8 + j) * pitch, 0));
+  };
+  auto store = [&](int buf, const float (&o)[8], const u32x4 (&x)[G::kA]) {
+    const Split8 s = split8(o);
+#pragma unroll
+    for (int p = 0; p < 3; ++p) sm.b[buf][p][kg][col] = s.part[p];
+#pragma unroll
+    for (int i = 0; i < G::kA; ++i) sm.a[buf][(int)threadIdx.x + kThreads * i] = x[i];
+  };
+
+  f32x16 acc[2][kNT];
+#pragma unroll
+  for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+    for (int nt = 0; nt < kNT; ++nt)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[mt][nt][r] = 0.0f;
+
+#pragma unroll
+  for (int i = 0; i < kPF; ++i) load(sb + i, wreg[i], areg[i]);
+  store(0, wreg[0], areg[0]);
+  wg_barrier();
+  // lane l of an operand holds row (column) l % 32 and k group l / 32
+  const int c0 = wc * 32 * kNT + (l & 31), r0 = (l >> 5) * BM + wr * 64 + (l & 31);
+  for (int s0 = sb; s0 < se; s0 += kPF) {
+#pragma unroll
+    for (int i = 0; i < kPF; ++i) {
+      const int buf = i & 1;  // kPF is even
+      load(s0 + i + kPF, wreg[i], areg[i]);  // these registers went to LDS one stage ago
+      u32x4 fa[2][3];
+#pragma unroll
+      for (int p = 0; p < 3; ++p)
+#pragma unroll
+        for (int mt = 0; mt < 2; ++mt) fa[mt][p] = sm.a[buf][2 * BM * p + r0 + 32 * mt];
+      // small products first
+      constexpr int pa[6] = {2, 0, 1, 1, 0, 0}, pb[6] = {0, 2, 1, 0, 1, 0};
+#pragma unroll
+      for (int nt = 0; nt < kNT; ++nt) {
+        u32x4 fb[3];
+#pragma unroll
+        for (int p = 0; p < 3; ++p) fb[p] = sm.b[buf][p][l >> 5][c0 + 32 * nt];
+#pragma unroll
+        for (int t = 0; t < 6; ++t)
+#pragma unroll
+          for (int mt = 0; mt < 2; ++mt)
+            acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, fa[mt][pa[t]]),
+                                                                  __builtin_bit_cast(bf16x8, fb[pb[t]]), acc[mt][nt],
+                                                                  0, 0, 0);
+      }
+      store(buf ^ 1, wreg[(i + 1) % kPF], areg[(i + 1) % kPF]);
+      wg_barrier();
+    }
+  }
+
+  // accumulator r of lane l holds row 8*(r/4) + 4*(l/32) + r%4, column l%32
+  const int nb = n0 + wr * 64 + 4 * (l >> 5), vb = v0 + c0;
+  auto row_of = [&](int mt, int r) { return nb + 32 * mt + 8 * (r >> 2) + (r & 3); };
+  bool redo = false;
+  if (gridDim.z == 1) {  // slices are checked where they are summed
+#pragma unroll
+    for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+      for (int nt = 0; nt < kNT; ++nt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          if (split_suspect(acc[mt][nt][r])) redo = redo || (row_of(mt, r) < a.N && vb + 32 * nt < V);
+  }
+  const bool f32 = __ballot(redo) != 0;
+  const HeadOut to = head_out(a);
+#pragma unroll
+  for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+    for (int nt = 0; nt < kNT; ++nt) {
+      const int v = vb + 32 * nt;
+      f32x16 y = acc[mt][nt];
+      if (f32) y = head_tile_f32(a, n0 + wr * 64 + 32 * mt, v0 + wc * 32 * kNT + 32 * nt);
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int n = row_of(mt, r);
+        if (n < a.N && v < V) to.p[(size_t)n * to.ld + v] = y[r];
+      }
+    }
+}
+
+// ------------------------------------------------------------ slices of k
+//
+// out = the slices' partial sums added in order.  SPLIT: an element that the
+// bf16 parts cannot carry is formed again in float32.
+template <bool SPLIT>
+__global__ __launch_bounds__(256) void k_head_sum(HeadArgs a, int slices) {
+  const int v = blockIdx.x * 256 + threadIdx.x, n = blockIdx.y;
+  if (v >= a.V) return;
+  const float* p = a.part + (size_t)n * a.V + v;
+  const size_t pitch = (size_t)a.N * a.V;
+  float s = 0.0f;
+#pragma unroll 8
+  for (int z = 0; z < slices; ++z) s += p[z * pitch];
+  if constexpr (SPLIT) {
+    if (split_suspect(s)) {
+      s = 0.0f;
+#pragma unroll 8
+      for (int k = 0; k < a.D; ++k) s = fmaf(split_act(a, n, k), a.w[(size_t)k * a.ldw + v], s);
+    }
+  }
+  a.out[(size_t)n * a.ldo + v] = s;
+}
+
+// ---------------------------------------------------------------- launch
+
+struct HeadPlan {
+  int rows;    // rows per workgroup: 16, 32 (k_head_skinny), 64, 128, 256 (k_head_split)
+  int slices;  // slices of k, each a workgroup of its own
+};
+
+// Microseconds a plan takes, to choose between plans: rounds of workgroups
+// times k steps times one step, but at least the read of W, plus the partial
+// sums' way through the caches.  The steps were measured at N 8 to 256 over
+// 4096 x 1000 (4 to 16 workgroups: a step's latency) and 4096 x 128 256 (every
+// CU at work: its throughput); over 54 sizes of (N, D, V) the plan this picks
+// is within 2% of the fastest of 20 in 46 of them, and within 16% in all.
+double plan_us(const HeadPlan& p, int N, int D, int V, int num_cu) {
+  const double w_bytes = 4.0 * D * V, rows = (N + p.rows - 1) / p.rows;
+  double us;
+  if (p.rows <= 32) {
+    const int kg = 256 / p.rows;  // k per group
+    const double steps = std::ceil((double)((D + kg - 1) / kg) / (kWaves * p.slices));
+    const double wgs = (double)((V + kSkinnyCols - 1) / kSkinnyCols) * rows * p.slices;
+    us = std::ceil(wgs / (2.0 * num_cu)) * steps * 1.1;  // two workgroups per CU
+    us = std::max(us, w_bytes / 5.4e6);
+  } else {
+    const int unit = p.rows == 256 ? 2 : 4;  // a slice is whole units of stages
+    const double steps = unit * std::ceil((double)((split_stages(D) + unit - 1) / unit) / p.slices);
+    const double wgs = (double)((V + kSplitCols - 1) / kSplitCols) * rows * p.slices;
+    if (p.rows == 64)  // one workgroup on a CU, or rounds of two
+      us = steps * (wgs <= num_cu ? 0.7 : 1.55 * std::ceil(wgs / (2.0 * num_cu)));
+    else
+      us = steps * (p.rows == 128 ? 1.4 : 2.3) * std::ceil(wgs / num_cu);
+    us = std::max(us, w_bytes / 4.4e6);
+  }
+  return p.slices > 1 ? us + 3.0 + 8.0 * p.slices * N * V / 5e6 : us;
+}
+
+// Rows per workgroup and slices of k.  Up to 32 rows the product is bound by
+// the read of W, not by the matrix cores (at 157 TFLOP/s 32 rows take half of
+// W's time in HBM), and k_head_skinny reads W at the rate of a copy; 33 rows
+// on would read it twice there (4096 x 128 256: 720 us for 17 rows in two tiles
+// of 16, 410 us in one of 32).  Slices fill the chip where the columns alone
+// do not (4096 x 1000, 8 rows: 44 us in one slice, 15 us in 16).
+HeadPlan head_plan(int N, int D, int V, int64_t ldw, int num_cu) {
+  const bool skinny = N <= 32 || ldw > kSplitMaxLdw;
+  const int lo = skinny ? (N <= 16 ? 16 : 32) : 64, hi = skinny ? lo : 256;
+  HeadPlan best{lo, 1};
+  double best_us = plan_us(best, N, D, V, num_cu);
+  for (int rows = lo; rows <= hi; rows *= 2)
+    for (int slices = 1; slices <= 32; slices *= 2) {
+      const HeadPlan p{rows, slices};
+      const double us = plan_us(p, N, D, V, num_cu);
+      if (us < best_us) {
+        best = p;
+        best_us = us;
+      }
+    }
+  return best;
+}
+
+size_t act_bytes(const HeadPlan& p, int N, int D) {
+  const size_t rows = ((size_t)N + p.rows - 1) / p.rows * p.rows;
+  return (size_t)split_stages(D) * kSplitK * rows * (p.rows <= 32 ? 4 : 6);
+}
+
+size_t head_ws_bytes(int N, int D, int V, int64_t ldw, int num_cu) {
+  const HeadPlan p = head_plan(N, D, V, ldw, num_cu);
+  return act_bytes(p, N, D) + 256 + (p.slices > 1 ? (size_t)p.slices * N * V * sizeof(float) : 0);
+}
+
 template <int R>
-hipError_t launch_head_skinny(const HeadArgs& a, hipStream_t s) {
+void launch_skinny(const HeadArgs& a, int slices, hipStream_t s) {
   hipLaunchKernelGGL(k_head_prep<R>, dim3(a.N), dim3(kThreads), 0, s, a);
-  const dim3 grid((unsigned)((a.V + kSkinnyCols - 1) / kSkinnyCols));
-  if (a.V < kSkinnyCols || a.ldw > (1 << 24)) hipLaunchKernelGGL((k_head_skinny<R, true>), grid, dim3(kThreads), 0, s, a);
+  const dim3 grid((unsigned)((a.V + kSkinnyCols - 1) / kSkinnyCols), (unsigned)((a.N + R - 1) / R), (unsigned)slices);
+  if (a.V < kSkinnyCols || a.ldw > kSplitMaxLdw) hipLaunchKernelGGL((k_head_skinny<R, true>), grid, dim3(kThreads), 0, s, a);
   else hipLaunchKernelGGL((k_head_skinny<R, false>), grid, dim3(kThreads), 0, s, a);
-  return hipGetLastError();
 }
 
-size_t head_ws_bytes(int N, int D) {
-  return ((size_t)head_kpad(D) * head_npad(N) + (size_t)N) * sizeof(float) + 256;
+template <int BM>
+void launch_split(HeadArgs a, int slices, hipStream_t s) {
+  const unsigned rt = (unsigned)((a.N + BM - 1) / BM);
+  a.lda = (int64_t)rt * BM;
+  hipLaunchKernelGGL(k_head_prep_split, dim3(a.N), dim3(kThreads), 0, s, a);
+  hipLaunchKernelGGL(k_head_split<BM>, dim3((unsigned)((a.V + kSplitCols - 1) / kSplitCols) * rt, 1, (unsigned)slices),
+                     dim3(kThreads), 0, s, a);
 }
 
-hipError_t launch_head(HeadArgs a, hipStream_t s) {
-  // up to 32 rows the product is bound by the one read of W, not by the
-  // matrix cores (at 157 TFLOP/s 32 rows take half of W's time in HBM)
-  if (a.N <= 16) return launch_head_skinny<16>(a, s);
-  if (a.N <= 32) return launch_head_skinny<32>(a, s);
-  // workspace: act [Dp][lda] (k-major), then rinv [N]
-  a.lda = head_npad(a.N);
-  a.rinv = a.act + (size_t)head_kpad(a.D) * a.lda;
-  hipLaunchKernelGGL(k_head_rms, dim3(a.N), dim3(kThreads), 0, s, a);
-  hipLaunchKernelGGL(k_head_act, dim3((unsigned)(head_kpad(a.D) / 32), (unsigned)(a.lda / 64)), dim3(kThreads), 0, s,
-                     a);
-  const dim3 grid((unsigned)((a.V + kHeadCols - 1) / kHeadCols), (unsigned)(a.lda / kHeadRows));
-  hipLaunchKernelGGL(k_head_gemm, grid, dim3(kGemmThreads), 0, s, a);
+hipError_t launch_head(HeadArgs a, int num_cu, hipStream_t s) {
+  const HeadPlan p = head_plan(a.N, a.D, a.V, a.ldw, num_cu);
+  a.part = reinterpret_cast<float*>(static_cast<char*>(a.act) + (act_bytes(p, a.N, a.D) + 255) / 256 * 256);
+  a.lda = (int64_t)((a.N + p.rows - 1) / p.rows) * p.rows;
+  switch (p.rows) {
+    case 16: launch_skinny<16>(a, p.slices, s); break;
+    case 32: launch_skinny<32>(a, p.slices, s); break;
+    case 64: launch_split<64>(a, p.slices, s); break;
+    case 128: launch_split<128>(a, p.slices, s); break;
+    default: launch_split<256>(a, p.slices, s); break;
+  }
+  if (p.slices > 1) {
+    const dim3 grid((unsigned)((a.V + 255) / 256), (unsigned)a.N);
+    if (p.rows <= 32) hipLaunchKernelGGL(k_head_sum<false>, grid, dim3(256), 0, s, a, p.slices);
+    else hipLaunchKernelGGL(k_head_sum<true>, grid, dim3(256), 0, s, a, p.slices);
+  }
   return hipGetLastError();
 }
 

@@ -143,9 +143,9 @@ struct HeadArgs {
   int64_t ldw;
   float* out;         // [N, ldo] logits
   int64_t ldo;
-  float* act;         // workspace [Dp, lda]: normalised rows, k-major, zero-padded
-  int64_t lda;
-  float* rinv;        // workspace [N]: 1 / rms of each row
+  void* act;          // workspace: the normalised rows in the product's operand layout
+  int64_t lda;        // rows of act (whole row tiles)
+  float* part;        // workspace [slices, N, V]: partial sums, with several slices of k
   int N, D, V;
 };
 
@@ -169,8 +169,8 @@ hipError_t launch_verify(const VerifyArgs& a, const VerifyWs& ws, bool f64, hipS
                          hipEvent_t between = nullptr);
 // Logits producer: workspace bytes (the normalised rows) and the two
 // launches (RMSNorm, then the MFMA product into out).
-size_t head_ws_bytes(int N, int D);
-hipError_t launch_head(HeadArgs a, hipStream_t s);
+size_t head_ws_bytes(int N, int D, int V, int64_t ldw, int num_cu);
+hipError_t launch_head(HeadArgs a, int num_cu, hipStream_t s);
 hipError_t launch_append(int32_t* slab, const int64_t* pos, const int32_t* ids, int n, hipStream_t s);
 
 }  // namespace plh

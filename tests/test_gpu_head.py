@@ -50,33 +50,67 @@ def test_head_matches_oracle(N, D, V):
     np.testing.assert_allclose(got, ref, rtol=1e-4, atol=1e-4)
 
 
-@pytest.mark.parametrize("N", [1, 16, 17, 32])          # the row counts at which the few-rows kernels change
+# (1, 16, 17, 32): the few-rows kernels; 33 on: the split kernels, with
+# ragged and whole row tiles.  A (D, V) pair reaches, as N grows, one and
+# several slices of k and every tile height.
+@pytest.mark.parametrize("N", [1, 16, 17, 32, 33, 64, 65, 129, 256])
 @pytest.mark.parametrize("D,V", [
-    (8, 127),    # one column short of a workgroup; k ends in a ragged group (16 rows) or a whole one (32)
-    (128, 128),  # one workgroup, whole groups, one k group per wave at 16 rows
-    (129, 129),  # the last workgroup's columns overlap the first's; one k past the whole groups
-    (1000, 333),
+    (8, 127),     # one column short of a workgroup; k ends in a ragged group (16 rows) or a whole one (32)
+    (128, 128),   # one workgroup, whole groups and stages
+    (129, 257),   # the last workgroup's columns overlap the one's before; one k past the whole groups
+    (1000, 333),  # several slices of k, the last one ragged
+    (40, 70000),  # enough columns for every tile height in one slice
 ])
-def test_few_rows(N, D, V):
-    """The few-rows kernels on W, h and out rows of odd strides (no 16-byte
-    alignment anywhere), nothing written outside out."""
+def test_row_counts_and_edges(N, D, V):
+    """Every kernel on W, h and out rows of odd strides (no 16-byte alignment
+    anywhere), nothing written outside out."""
     import torch
 
-    print(f"[head] few rows N={N} D={D} V={V}", flush=True)
+    print(f"[head] edges N={N} D={D} V={V}", flush=True)
     h, norm, W = _case(N + D, N, D, V)
     wb = torch.full((D, V + 3), float("nan"), device="cuda")
     wb[:, 1:V + 1] = torch.from_numpy(W).cuda()
     hb = torch.full((N, D + 1), float("nan"), device="cuda")
     hb[:, :D] = torch.from_numpy(h).cuda()
     ob = torch.full((N + 1, V + 5), 7.0, device="cuda")
-    torch.cuda.synchronize()
     H.rms_norm_lm_head(hb[:, :D], torch.from_numpy(norm).cuda(), wb[:, 1:V + 1], 1e-5, out=ob[:N, :V])
-    torch.cuda.synchronize()
     got = ob.cpu().numpy()
     bound = oracle.head_error_bound(h, norm, W, 1e-5)
     err = np.abs(got[:N, :V].astype(np.float64) - oracle.lm_head_logits(h, norm, W, 1e-5))
     assert np.all(err <= TOL * bound + 1e-30), float(np.max(err / (bound + 1e-30)))
     assert np.all(got[N:] == 7.0) and np.all(got[:, V:] == 7.0)
+
+
+@pytest.mark.parametrize("N", [8, 40])  # the fp32 kernel and the bf16 split
+@pytest.mark.parametrize("D,V", [(64, 70000), (512, 300)])  # one slice of k, and several
+def test_values_at_the_ends_of_float32(N, D, V):
+    """Infinities, NaN, values next to overflow and subnormal-sized results:
+    the same kinds of value as float32 products and sums give."""
+    h, norm, W = _case(5, N, D, V)
+    W[3, 7] = np.inf        # +-inf in column 7
+    W[4, 9], W[5, 9] = np.inf, -np.inf   # inf - inf somewhere in column 9
+    W[:, 11] = 3.3e38       # overflows on the way for some rows
+    W[:, 13] *= np.float32(1e-36)   # tiny: its bf16 parts underflow
+    W[:, 14] = 0.0
+    h[2, 1] = np.nan        # a whole NaN row
+    got = H.rms_norm_lm_head(h, norm, W, 1e-5)
+    with np.errstate(all="ignore"):
+        a = oracle.rms_norm(h, norm, np.float32(1e-5)).astype(np.float64)
+        ref = a @ W.astype(np.float64)
+    ok = np.arange(N) != 2
+    assert np.isnan(got[2]).all() and np.isfinite(got[ok][:, :7]).all()
+    assert np.array_equal(got[ok, 7], np.sign(a[ok, 3]) * np.inf)
+    same = np.sign(a[ok, 4]) != np.sign(a[ok, 5])
+    assert np.array_equal(got[ok, 9][same], (np.sign(a[ok, 4]) * np.inf)[same]) and np.isnan(got[ok, 9][~same]).all()
+    over = np.abs(ref[ok, 11]) > 3.5e38  # float32's largest is 3.40e38; partial sums of the rest may overflow too
+    assert not np.isfinite(got[ok, 11][over]).any()
+    bound = np.abs(a) @ np.abs(W.astype(np.float64))
+    # a product of 1e-38 is rounded to float32's subnormal step, 2^-149
+    assert np.all(np.abs(got[ok, 13] - ref[ok, 13]) <= TOL * bound[ok, 13] + D * 2.0 ** -149)
+    assert np.all(got[ok, 14] == 0.0)
+    rest = np.setdiff1d(np.arange(V), [7, 9, 11, 13, 14])
+    err = np.abs(got[ok][:, rest] - ref[ok][:, rest])
+    assert np.all(err <= TOL * bound[ok][:, rest] + 1e-30)
 
 
 def test_tiny_rows_and_eps():
