@@ -520,7 +520,21 @@ int plh_draw(plh_ctx* c, const void* p, int dtype, int64_t ld, int B, int V, con
     return fail(c, PLH_ERR_INVALID_ARG, "null device pointer%s");
   int rc = use_device(c);
   if (rc != PLH_OK) return rc;
-  plh::DrawArgs a{p, ld, B, V, uniforms, out_ids};
+  plh::DrawArgs a{p, ld, B, V, uniforms, out_ids, nullptr};
+  const size_t need = plh::draw_ws_bytes(B, V, c->num_cu);
+  if (need > 0) {
+    // the one-launch form needs no workspace: it serves calls under graph
+    // capture, which must not allocate or wait for another stream
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    PLH_HIP(c, hipStreamIsCapturing(c->stream, &st), "hipStreamIsCapturing");
+    if (st == hipStreamCaptureStatusNone) {
+      rc = reserve_ws(c, need);
+      if (rc != PLH_OK) return rc;
+      a.sums = static_cast<double*>(c->ws);
+      c->ws_stream = c->stream;
+      c->ws_open = true;
+    }
+  }
   const hipError_t e = plh::launch_draw(a, dtype == PLH_F64, c->stream);
   if (e != hipSuccess) return hip_fail(c, e, "plh_draw launch");
   return PLH_OK;

@@ -103,6 +103,7 @@ struct DrawArgs {
   int B, V;
   const double* uniforms;
   int32_t* out_ids;
+  double* sums;  // workspace: the rows' piece sums (two launches), or null (one)
 };
 
 struct PenalizeArgs {
@@ -158,6 +159,8 @@ ChunkWs fast_ws_layout(void* base, int B, int V, bool f64);
 // not null, is recorded on s between the two kernels.
 hipError_t launch_sample_fast(const SampleArgs& a, bool f64, bool vec, int num_cu, hipStream_t s,
                               hipEvent_t between = nullptr);
+// Draw: workspace bytes (0: one launch, none needed), and the launches.
+size_t draw_ws_bytes(int B, int V, int num_cu);
 hipError_t launch_draw(const DrawArgs& a, bool f64, hipStream_t s);
 hipError_t launch_penalize(const PenalizeArgs& a, bool f64, hipStream_t s);
 // Verify: workspace bytes for B rows of V tokens, its layout, and the two

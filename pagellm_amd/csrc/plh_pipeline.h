@@ -430,58 +430,6 @@ __device__ __forceinline__ SelResult value_select(const Visit& visit, double zlo
   return sorted_pick<MODE>(target, above, sm);
 }
 
-// ----------------------------------------------------------------- draw
-
-// Inverse-CDF draw over non-negative weights w(i), i < V (sampling.py:94-98):
-// the first i whose running mass exceeds u * total, else V - 1.  Weights are
-// normalised by their float64 total, then summed exactly in fixed point.
-template <class W>
-__device__ __forceinline__ int draw_weights(const W& wfn, int V, double u, double* redd, uint64_t* redu, int* redi) {
-  double s = 0.0;
-  for (int base = 0; base < V; base += (4 * kThreads))
-#pragma unroll
-    for (int l = 0; l < 4; ++l) {
-      const int i = base + 4 * (int)threadIdx.x + l;
-      if (i < V) s += wfn(i);
-    }
-  const double Wt = block_sum(s, redd);
-  if (!(Wt > 0.0)) return V - 1;
-  uint64_t tf = 0;
-  for (int base = 0; base < V; base += (4 * kThreads))
-#pragma unroll
-    for (int l = 0; l < 4; ++l) {
-      const int i = base + 4 * (int)threadIdx.x + l;
-      if (i < V) tf += to_fx(wfn(i) / Wt);
-    }
-  tf = block_sum<uint64_t>(tf, redu);
-  const uint64_t t_fx = (uint64_t)__double2ull_rd(u * (double)tf);
-  uint64_t run = 0;
-  for (int base = 0; base < V; base += (4 * kThreads)) {
-    uint64_t w[4], ts = 0;
-#pragma unroll
-    for (int l = 0; l < 4; ++l) {
-      const int i = base + 4 * (int)threadIdx.x + l;
-      w[l] = i < V ? to_fx(wfn(i) / Wt) : 0ull;
-      ts += w[l];
-    }
-    uint64_t tt;
-    const uint64_t ex = block_excl_scan<uint64_t>(ts, redu, &tt);
-    if (run + tt > t_fx) {
-      uint64_t c = run + ex;
-      int my = INT_MAX;
-#pragma unroll
-      for (int l = 0; l < 4; ++l) {
-        c += w[l];
-        if (my == INT_MAX && c > t_fx) my = base + 4 * (int)threadIdx.x + l;
-      }
-      const int f = block_min<int>(my, redi);
-      return f == INT_MAX ? V - 1 : f;
-    }
-    run += tt;
-  }
-  return V - 1;
-}
-
 // ------------------------------------------------------------- pipeline
 
 struct PipeIn {

@@ -3279,23 +3279,6 @@ __global__ __launch_bounds__(kThreads) void k_nuc_final(SampleArgs a) {
   if (threadIdx.x == 0) a.out_ids[row] = id;
 }
 
-// ------------------------------------------------------------------- draw
-
-template <typename TIn>
-__global__ __launch_bounds__(kThreads) void k_draw(DrawArgs a) {
-  __shared__ double redd[kWaves];
-  __shared__ uint64_t redu[kWaves];
-  __shared__ int redi[kWaves];
-  const int row = blockIdx.x;
-  const TIn* p = reinterpret_cast<const TIn*>(a.p) + (int64_t)row * a.ld;
-  auto w = [&](int i) -> double {
-    const double v = (double)p[i];
-    return v > 0.0 ? v : 0.0;
-  };
-  const int id = draw_weights(w, a.V, a.uniforms[row], redd, redu, redi);
-  if (threadIdx.x == 0) a.out_ids[row] = id;
-}
-
 // --------------------------------------------------------------- penalize
 
 // apply_repetition_penalty on a copy (sampling.py:52-62), in the input's
@@ -3451,12 +3434,6 @@ hipError_t launch_sample_fast(const SampleArgs& a, bool f64, bool vec, int num_c
 
 hipError_t launch_append(int32_t* slab, const int64_t* pos, const int32_t* ids, int n, hipStream_t s) {
   hipLaunchKernelGGL(k_append, dim3((n + 255) / 256), dim3(256), 0, s, slab, pos, ids, n);
-  return hipGetLastError();
-}
-
-hipError_t launch_draw(const DrawArgs& a, bool f64, hipStream_t s) {
-  if (f64) hipLaunchKernelGGL((k_draw<double>), dim3(a.B), dim3(kThreads), 0, s, a);
-  else hipLaunchKernelGGL((k_draw<float>), dim3(a.B), dim3(kThreads), 0, s, a);
   return hipGetLastError();
 }
 

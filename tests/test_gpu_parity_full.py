@@ -160,3 +160,60 @@ def test_small_batch_at_a_large_vocabulary(dtype):
     w["logits"] = w["logits"].astype(dtype)
     ids = sample_batch(w["logits"], w["params"], uniforms=w["uniforms"], contexts=w["contexts"])
     _compare_rows(w, range(16), ids, f"mixed128k x16 {np.dtype(dtype).name}")
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("V", [1, 511, 512, 513, 4608, 4609, 40000, 40001, 49153])
+def test_draw_piece_and_launch_edges(V, dtype):
+    """Rows around the 512-token pieces, the waves' shares (8 pieces and a
+    remainder) and the vocabulary from which few rows take two launches:
+    spread mass, mass in one token of each piece, mass at the two ends."""
+    g = np.random.default_rng(V)
+    p = g.random((6, V)).astype(dtype)
+    p[1] = 0
+    p[1, ::509] = 1
+    p[2, 1:-1] = 0
+    p[3] = 0
+    p[3, g.integers(V)] = 2.5
+    p[4] = -p[4]       # nothing positive: the last id
+    p[5, V // 2:] = 0  # u next to 1 must not pass the last positive token
+    u = g.random(6)
+    u[5] = 1 - 2.0 ** -53
+    ids = draw_batch(p, u)
+    for b in (0, 1, 2, 3, 5):
+        ref = oracle.draw(p[b].astype(np.float64), float(u[b]))
+        if b == 5 and V > 1:  # the oracle's u * total may round to the total; a positive token either way
+            last = int(np.flatnonzero(p[b] > 0)[-1])
+            assert ids[b] == last and ref in (last, V - 1)
+        elif ids[b] != ref:
+            assert oracle.draw_boundary_gap(p[b].astype(np.float64), float(u[b])) < 1e-12, (b, ids[b], ref)
+    assert ids[4] == V - 1
+
+
+def test_draw_under_graph_capture():
+    """A draw whose eager form uses the workspace is captured and replayed
+    with new inputs."""
+    import torch
+
+    from pagellm_amd import _native
+
+    V, B = 50257, 3
+    p = torch.rand((B, V), device="cuda", dtype=torch.float64)
+    u = torch.rand(B, device="cuda", dtype=torch.float64)
+    ids = torch.zeros(B, device="cuda", dtype=torch.int32)
+    c = _native.Context(0)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        c.set_stream(torch.cuda.current_stream().cuda_stream)
+        c.draw(p.data_ptr(), _native.PLH_F64, V, B, V, u.data_ptr(), ids.data_ptr())
+    for seed in range(3):
+        g = np.random.default_rng(seed)
+        hp, hu = g.random((B, V)) ** 4, g.random(B)
+        p.copy_(torch.from_numpy(hp))
+        u.copy_(torch.from_numpy(hu))
+        graph.replay()
+        torch.cuda.synchronize()
+        ref = [oracle.draw(hp[b], float(hu[b])) for b in range(B)]
+        assert ids.tolist() == ref == draw_batch(hp, hu).tolist()
+    c.set_stream(None)
