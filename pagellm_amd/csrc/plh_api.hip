@@ -205,8 +205,10 @@ int sample_impl(plh_ctx* c, const void* logits, int dtype, int64_t ld, int B, in
   a.nucleus_only = a.nucleus && (flags & PLH_SAMPLE_NUCLEUS_ONLY) ? 1 : 0;
   const bool f64 = dtype == PLH_F64;
   // the fast path gathers per-row state in LDS sized for V <= 262144
+  const bool small = V <= plh::kSmallV && !(flags & PLH_SAMPLE_ROWWISE);  // one launch, no workspace
   if (out_probs != nullptr || (flags & PLH_SAMPLE_ROWWISE) || V > kMaxVBitmap) {
-    const hipError_t e = plh::launch_sample_rows(a, f64, vec, c->stream);
+    const hipError_t e = small ? plh::launch_sample_small(a, f64, c->stream, nullptr)
+                               : plh::launch_sample_rows(a, f64, vec, c->stream);
     if (e != hipSuccess) return hip_fail(c, e, "plh_sample launch");
     return PLH_OK;
   }
@@ -221,23 +223,29 @@ int sample_impl(plh_ctx* c, const void* logits, int dtype, int64_t ld, int B, in
     rc = order_scratch(c);
     if (rc != PLH_OK) return rc;
     a.ws = plh::fast_ws_layout(c->scratch, B, V, f64);
-    const hipError_t e = plh::launch_sample_fast(a, f64, vec, c->num_cu, c->stream, nullptr);
+    const hipError_t e = small ? plh::launch_sample_small(a, f64, c->stream, nullptr)
+                               : plh::launch_sample_fast(a, f64, vec, c->num_cu, c->stream, nullptr);
     if (e != hipSuccess) return hip_fail(c, e, "plh_sample_noalloc launch");
     c->scratch_stream = c->stream;
     c->scratch_open = true;
     return PLH_OK;
   }
-  rc = reserve_ws(c, need);
-  if (rc != PLH_OK) return rc;
-  a.ws = plh::fast_ws_layout(c->ws, B, V, f64);
+  if (!small) {
+    rc = reserve_ws(c, need);
+    if (rc != PLH_OK) return rc;
+    a.ws = plh::fast_ws_layout(c->ws, B, V, f64);
+  }
   std::array<hipEvent_t, 3> ev{};
   rc = timing_begin(c, ev);
   if (rc != PLH_OK) return rc;
-  const hipError_t e = plh::launch_sample_fast(a, f64, vec, c->num_cu, c->stream, ev[1]);
+  const hipError_t e = small ? plh::launch_sample_small(a, f64, c->stream, ev[1])
+                             : plh::launch_sample_fast(a, f64, vec, c->num_cu, c->stream, ev[1]);
   if (e != hipSuccess) return hip_fail(c, e, "plh_sample launch");
   if (c->timing) PLH_HIP(c, hipEventRecord(ev[2], c->stream), "hipEventRecord");
-  c->ws_stream = c->stream;
-  c->ws_open = true;
+  if (!small) {
+    c->ws_stream = c->stream;
+    c->ws_open = true;
+  }
   return PLH_OK;
 }
 

@@ -150,6 +150,10 @@ struct HeadArgs {
   int N, D, V;
 };
 
+// Rows of at most kSmallV tokens: the whole call in one launch, no workspace.
+// `between` (when not null) is recorded after it.
+constexpr int kSmallV = 2048;
+hipError_t launch_sample_small(const SampleArgs& a, bool f64, hipStream_t s, hipEvent_t between);
 hipError_t launch_sample_rows(const SampleArgs& a, bool f64, bool vec, hipStream_t s);
 // Fast path: workspace bytes for a [B, V] batch, its layout inside `base`
 // (256-byte aligned), and the two launches.

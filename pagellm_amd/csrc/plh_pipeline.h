@@ -19,6 +19,7 @@
 
 #include "plh_device.h"
 #include "plh_fast.h"
+#include "plh_kernels.h"
 
 namespace plh {
 
@@ -51,6 +52,70 @@ struct RowParams {
   bool nucleus;  // the row takes the nucleus path of the fast kernels
 };
 
+constexpr double kNucTopP = 0.98;  // top_p from which a row may take the nucleus path
+
+__device__ __forceinline__ RowParams load_row_params(const SampleArgs& a, int row) {
+  RowParams rp;
+  rp.T = a.temperature[row];
+  rp.top_k = a.top_k[row];
+  rp.top_p = a.top_p[row];
+  rp.pen = a.rep_penalty[row];
+  rp.u = a.uniforms != nullptr ? a.uniforms[row] : 0.0;
+  rp.h0 = a.hist_off != nullptr ? a.hist_off[a.hist_spans ? 2 * row : row] : 0;
+  rp.h1 = a.hist_off != nullptr ? a.hist_off[a.hist_spans ? 2 * row + 1 : row + 1] : 0;
+  rp.greedy = rp.T == 0.0;  // SamplingParams.greedy (sampling.py:47-49)
+  // sampling.py:56: no penalty when it is 1.0 or the context is empty
+  rp.pen_active = rp.pen != 1.0 && rp.h1 > rp.h0 && a.hist_ids != nullptr;
+  rp.topk = !rp.greedy && rp.top_k > 0 && rp.top_k < a.V;  // :76
+  rp.topp = !rp.greedy && rp.top_p < 1.0;                  // :82
+  rp.nucleus = a.nucleus != 0 && rp.topp && !rp.topk && rp.top_p >= kNucTopP;
+  return rp;
+}
+
+// The same parameters read with vector loads (every lane the same
+// address), so that they travel in one round trip with the other loads a
+// kernel issues before it knows the row's mode; row_params_of() makes them
+// uniform once they are in.
+struct RowLoad {
+  double T, top_p, pen, u;
+  int top_k;
+  int64_t h0, h1;
+};
+
+__device__ __forceinline__ int lane_zero() {
+  int z;
+  asm volatile("v_mov_b32 %0, 0" : "=v"(z));  // a zero the compiler cannot see as uniform
+  return z;
+}
+
+__device__ __forceinline__ void issue_row_params(const SampleArgs& a, int row, RowLoad& rl) {
+  const int r = row + lane_zero();
+  rl.T = a.temperature[r];
+  rl.top_k = a.top_k[r];
+  rl.top_p = a.top_p[r];
+  rl.pen = a.rep_penalty[r];
+  rl.u = a.uniforms != nullptr ? a.uniforms[r] : 0.0;
+  rl.h0 = a.hist_off != nullptr ? a.hist_off[a.hist_spans ? 2 * r : r] : 0;
+  rl.h1 = a.hist_off != nullptr ? a.hist_off[a.hist_spans ? 2 * r + 1 : r + 1] : 0;
+}
+
+__device__ __forceinline__ RowParams row_params_of(const SampleArgs& a, const RowLoad& rl) {
+  RowParams rp;
+  rp.T = uniform(rl.T);
+  rp.top_k = uniform(rl.top_k);
+  rp.top_p = uniform(rl.top_p);
+  rp.pen = uniform(rl.pen);
+  rp.u = uniform(rl.u);
+  rp.h0 = (int64_t)uniform((uint64_t)rl.h0);
+  rp.h1 = (int64_t)uniform((uint64_t)rl.h1);
+  rp.greedy = rp.T == 0.0;
+  rp.pen_active = rp.pen != 1.0 && rp.h1 > rp.h0 && a.hist_ids != nullptr;
+  rp.topk = !rp.greedy && rp.top_k > 0 && rp.top_k < a.V;
+  rp.topp = !rp.greedy && rp.top_p < 1.0;
+  rp.nucleus = a.nucleus != 0 && rp.topp && !rp.topk && rp.top_p >= kNucTopP;
+  return rp;
+}
+
 // sampling.py:59-61: divide positive logits, multiply the others.
 __device__ __forceinline__ double penalize(double x, double pen) { return x > 0.0 ? x / pen : x * pen; }
 
@@ -78,6 +143,21 @@ struct PCalc {
 __device__ __forceinline__ double p_of(const PCalc& c, double z) {
   if (!(z >= c.z_lo)) return 0.0;
   return fast_exp_neg(z * c.invT - c.ymax, c.tab) * c.invS;
+}
+
+// The smallest z that top-k keeps, from the k-th largest: the one whose
+// y = z / T still reaches the k-th's (division can merge neighbouring values;
+// a few steps at most).
+__device__ __forceinline__ double topk_floor(double kth_z, double T) {
+  if (!(kth_z > -INFINITY)) return -INFINITY;
+  const double kth_y = (T == 1.0) ? kth_z : kth_z / T;
+  double z_lo = kth_z;
+  for (int it = 0; it < 64; ++it) {
+    const double zp = dbl_prev(z_lo);
+    const double yp = (T == 1.0) ? zp : zp / T;
+    if (yp >= kth_y) z_lo = zp; else break;
+  }
+  return z_lo;
 }
 
 // ------------------------------------------------------------ source
@@ -495,17 +575,7 @@ __device__ __forceinline__ int row_pipeline(Src& src, const RowParams& rp, int V
     };
     const SelResult r = value_select<kCount>(visit, zmin, zmax, (uint64_t)rp.top_k, sm);
     const double kth_z = val_of_key(r.key);
-    if (kth_z > -INFINITY) {
-      const double kth_y = (T == 1.0) ? kth_z : kth_z / T;
-      z_lo = kth_z;
-      // smallest z whose y = z / T still reaches kth_y (division can merge
-      // neighbouring values); a few steps at most
-      for (int it = 0; it < 64; ++it) {
-        const double zp = dbl_prev(z_lo);
-        const double yp = (T == 1.0) ? zp : zp / T;
-        if (yp >= kth_y) z_lo = zp; else break;
-      }
-    }
+    z_lo = topk_floor(kth_z, T);
   }
 
   // ---- softmax normaliser over the survivors (:79-81)

@@ -112,7 +112,6 @@ constexpr int kHBuf = 3;          // rotating histogram buffers of the merge
 constexpr int kDrawSpanMax = 256; // tokens per draw bin, at most (V <= 262144)
 constexpr int kSegPerLane = 8;    // segments per lane of one wave (V <= 262144)
 constexpr int kHistBatch = 8;     // history ids a thread loads at once
-constexpr double kNucTopP = 0.98; // top_p from which a row may take the nucleus path
 
 // Chunk geometry per input type: a wave-wide 16-byte load covers kSpan
 // consecutive tokens, a wave owns one contiguous segment of kSeg tokens and
@@ -161,68 +160,6 @@ union SmemAll {
   Smem g;
 };
 
-
-__device__ __forceinline__ RowParams load_row_params(const SampleArgs& a, int row) {
-  RowParams rp;
-  rp.T = a.temperature[row];
-  rp.top_k = a.top_k[row];
-  rp.top_p = a.top_p[row];
-  rp.pen = a.rep_penalty[row];
-  rp.u = a.uniforms != nullptr ? a.uniforms[row] : 0.0;
-  rp.h0 = a.hist_off != nullptr ? a.hist_off[a.hist_spans ? 2 * row : row] : 0;
-  rp.h1 = a.hist_off != nullptr ? a.hist_off[a.hist_spans ? 2 * row + 1 : row + 1] : 0;
-  rp.greedy = rp.T == 0.0;  // SamplingParams.greedy (sampling.py:47-49)
-  // sampling.py:56: no penalty when it is 1.0 or the context is empty
-  rp.pen_active = rp.pen != 1.0 && rp.h1 > rp.h0 && a.hist_ids != nullptr;
-  rp.topk = !rp.greedy && rp.top_k > 0 && rp.top_k < a.V;  // :76
-  rp.topp = !rp.greedy && rp.top_p < 1.0;                  // :82
-  rp.nucleus = a.nucleus != 0 && rp.topp && !rp.topk && rp.top_p >= kNucTopP;
-  return rp;
-}
-
-// The same parameters read with vector loads (every lane the same
-// address), so that they travel in one round trip with the other loads a
-// kernel issues before it knows the row's mode; row_params_of() makes them
-// uniform once they are in.
-struct RowLoad {
-  double T, top_p, pen, u;
-  int top_k;
-  int64_t h0, h1;
-};
-
-__device__ __forceinline__ int lane_zero() {
-  int z;
-  asm volatile("v_mov_b32 %0, 0" : "=v"(z));  // a zero the compiler cannot see as uniform
-  return z;
-}
-
-__device__ __forceinline__ void issue_row_params(const SampleArgs& a, int row, RowLoad& rl) {
-  const int r = row + lane_zero();
-  rl.T = a.temperature[r];
-  rl.top_k = a.top_k[r];
-  rl.top_p = a.top_p[r];
-  rl.pen = a.rep_penalty[r];
-  rl.u = a.uniforms != nullptr ? a.uniforms[r] : 0.0;
-  rl.h0 = a.hist_off != nullptr ? a.hist_off[a.hist_spans ? 2 * r : r] : 0;
-  rl.h1 = a.hist_off != nullptr ? a.hist_off[a.hist_spans ? 2 * r + 1 : r + 1] : 0;
-}
-
-__device__ __forceinline__ RowParams row_params_of(const SampleArgs& a, const RowLoad& rl) {
-  RowParams rp;
-  rp.T = uniform(rl.T);
-  rp.top_k = uniform(rl.top_k);
-  rp.top_p = uniform(rl.top_p);
-  rp.pen = uniform(rl.pen);
-  rp.u = uniform(rl.u);
-  rp.h0 = (int64_t)uniform((uint64_t)rl.h0);
-  rp.h1 = (int64_t)uniform((uint64_t)rl.h1);
-  rp.greedy = rp.T == 0.0;
-  rp.pen_active = rp.pen != 1.0 && rp.h1 > rp.h0 && a.hist_ids != nullptr;
-  rp.topk = !rp.greedy && rp.top_k > 0 && rp.top_k < a.V;
-  rp.topp = !rp.greedy && rp.top_p < 1.0;
-  rp.nucleus = a.nucleus != 0 && rp.topp && !rp.topk && rp.top_p >= kNucTopP;
-  return rp;
-}
 
 template <typename TIn, bool VEC>
 __device__ __forceinline__ int row_general(const SampleArgs& a, int row, const RowParams& rp, Smem& sm,
