@@ -132,8 +132,8 @@ int plh_sync(plh_ctx* ctx);
  *               of :98); ignored for greedy rows
  *   out_ids     int32 [B]    sampled token ids
  *   out_probs   float64 [B, V] or NULL: when given, the processed
- *               distribution (probs(), :65-91) is written too and the
- *               row-wise kernel is used
+ *               distribution (probs(), :65-91) is written too, by
+ *               one workgroup per row and without any workspace
  *   flags       PLH_SAMPLE_* bits
  * Histories with an active penalty require V <= 262144.
  */

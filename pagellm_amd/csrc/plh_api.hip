@@ -207,8 +207,10 @@ int sample_impl(plh_ctx* c, const void* logits, int dtype, int64_t ld, int B, in
   // the fast path gathers per-row state in LDS sized for V <= 262144
   const bool small = V <= plh::kSmallV && !(flags & PLH_SAMPLE_ROWWISE);  // one launch, no workspace
   if (out_probs != nullptr || (flags & PLH_SAMPLE_ROWWISE) || V > kMaxVBitmap) {
-    const hipError_t e = small ? plh::launch_sample_small(a, f64, c->stream, nullptr)
-                               : plh::launch_sample_rows(a, f64, vec, c->stream);
+    const bool probs = out_probs != nullptr && V <= plh::kProbsV && !(flags & PLH_SAMPLE_ROWWISE);
+    const hipError_t e = small   ? plh::launch_sample_small(a, f64, c->stream, nullptr)
+                         : probs ? plh::launch_probs_rows(a, f64, c->stream)
+                                 : plh::launch_sample_rows(a, f64, vec, c->stream);
     if (e != hipSuccess) return hip_fail(c, e, "plh_sample launch");
     return PLH_OK;
   }

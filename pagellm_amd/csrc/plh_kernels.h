@@ -154,6 +154,10 @@ struct HeadArgs {
 // `between` (when not null) is recorded after it.
 constexpr int kSmallV = 2048;
 hipError_t launch_sample_small(const SampleArgs& a, bool f64, hipStream_t s, hipEvent_t between);
+// The processed distributions (and ids) of rows of kSmallV + 1 to kProbsV
+// tokens: one launch, no workspace.
+constexpr int kProbsV = 262144;
+hipError_t launch_probs_rows(const SampleArgs& a, bool f64, hipStream_t s);
 hipError_t launch_sample_rows(const SampleArgs& a, bool f64, bool vec, hipStream_t s);
 // Fast path: workspace bytes for a [B, V] batch, its layout inside `base`
 // (256-byte aligned), and the two launches.
