@@ -292,6 +292,18 @@ __device__ __forceinline__ TIn in_min3(TIn a, TIn b, TIn c) {
     return fmin(fmin(a, b), c);
   }
 }
+// v, or NaN (which in_min3 passes over) for an infinity: v * 0 + v, one
+// instruction where a compare and a select take two.
+__device__ __forceinline__ float finite_or_nan(float v) {
+  float r;
+  asm("v_fma_f32 %0, %1, 0, %1" : "=v"(r) : "v"(v));
+  return r;
+}
+__device__ __forceinline__ double finite_or_nan(double v) {
+  double r;
+  asm("v_fma_f64 %0, %1, 0, %1" : "=v"(r) : "v"(v));
+  return r;
+}
 // (m1, m2): the largest two values seen (m1 >= m2), then x
 template <typename TIn>
 __device__ __forceinline__ void in_top2(TIn& m1, TIn& m2, TIn x) {
@@ -459,6 +471,26 @@ struct ChunkToks {
   __device__ __forceinline__ int pen_tok(const ChunkSmem& cm, int i) const { return cm.pt[wave()][lane() + kWave * i]; }
 };
 
+// v where bit e of pb is clear, -inf where it is set: two instructions a
+// register and no branch.
+template <int E>
+__device__ __forceinline__ float drop_slot(float v, uint32_t pb, uint32_t ninf) {
+  const uint32_t m = (uint32_t)((int32_t)(pb << (31 - E)) >> 31);  // v_bfe_i32
+  return __uint_as_float((m & ninf) | (~m & __float_as_uint(v)));  // v_bfi_b32
+}
+template <int E>
+__device__ __forceinline__ double drop_slot(double v, uint32_t pb, uint32_t) {
+  return ((pb >> E) & 1u) ? -INFINITY : v;
+}
+template <typename TIn, int E>
+__device__ __forceinline__ void drop_slots(ChunkToks<TIn>& tk, uint32_t pb, uint32_t ninf) {
+  using G = Geo<TIn>;
+  if constexpr (E < G::kEpt) {
+    tk.v[E / G::kVW][E % G::kVW] = drop_slot<E>(tk.rv(E), pb, ninf);
+    drop_slots<TIn, E + 1>(tk, pb, ninf);
+  }
+}
+
 // Moves the calling wave's penalised tokens (bits pb of each lane) out of
 // the registers: their penalised float64 value goes to the wave's LDS pool,
 // the register slot to -inf.  Every lane then takes its share of the pool
@@ -466,25 +498,47 @@ struct ChunkToks {
 // set (its registers or its share of the pool), so per-lane maxima stay
 // maxima of disjoint sets.  Returns true when the pool overflows (the chunk
 // is then incomplete).
+//
+// A lane has few penalised tokens (0.4 of 32 with 2000 distinct ids in 152 064)
+// but some lane of the wave has one in most slots, so a branch per slot ran
+// nearly all of the bodies; the tokens are read again from the row (x) instead,
+// kPenBatch at a time, by their set bits.
+constexpr int kPenBatch = 4;
 template <typename TIn>
-__device__ __forceinline__ bool set_aside_penalised(ChunkToks<TIn>& tk, uint32_t pb, double pen, int c0, ChunkSmem& cm) {
+__device__ __forceinline__ bool set_aside_penalised(ChunkToks<TIn>& tk, uint32_t pb, double pen, int c0, const TIn* x,
+                                                    ChunkSmem& cm) {
   using G = Geo<TIn>;
   const int n = __popc(pb);
   const int incl = wave_scan_incl(n, 0, OpAdd{});
   const int total = lane_value(incl, kWave - 1);
   tk.np = 0;
   if (total > kPenPerWave) return true;
-  if (pb != 0u) {
-    int k = incl - n;
+  uint32_t ninf = 0xff800000u;
+  asm volatile("" : "+v"(ninf));  // a register: v_bfi_b32 takes no literal
+  drop_slots<TIn, 0>(tk, pb, ninf);
+  const int q0 = c0 + wave() * G::kSeg + lane() * G::kVW;
+  int k = incl - n;
+  for (uint32_t m = pb; m != 0u;) {
+    TIn z[kPenBatch];
+    int tok[kPenBatch];
 #pragma unroll
-    for (int e = 0; e < G::kEpt; ++e) {
-      if ((pb >> e) & 1u) {
-        cm.pz[wave()][k] = tk.raw(e);
-        cm.pt[wave()][k] = c0 + slot_q<TIn>(e);
-        ++k;
-        tk.v[e / G::kVW][e % G::kVW] = (TIn)(-INFINITY);
+    for (int i = 0; i < kPenBatch; ++i) {
+      tok[i] = -1;
+      if (m != 0u) {
+        const int e = __builtin_ctz(m);
+        m &= m - 1u;
+        tok[i] = q0 + (e / G::kVW) * G::kSpan + e % G::kVW;
       }
     }
+#pragma unroll
+    for (int i = 0; i < kPenBatch; ++i) z[i] = x[max(tok[i], 0)];
+#pragma unroll
+    for (int i = 0; i < kPenBatch; ++i)
+      if (tok[i] >= 0) {
+        cm.pz[wave()][k] = (double)z[i];
+        cm.pt[wave()][k] = tok[i];
+        ++k;
+      }
   }
   // the lane's share (a wave's own LDS writes complete in order), penalised
   // with one division each
@@ -974,7 +1028,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
   int flags = 0;
   if (rp.pen_active) {
     const uint32_t pb = chunk_pbits<TIn>(a, rp, c0, cm);
-    if (set_aside_penalised<TIn>(tk, pb, rp.pen, c0, cm)) flags = kChunkIncomplete;
+    if (set_aside_penalised<TIn>(tk, pb, rp.pen, c0, x, cm)) flags = kChunkIncomplete;
     if (NUC && rp.nucleus) {  // the nucleus kernels read the chunk's bitmap from here
       uint32_t* out = a.ws.npen + (size_t)g * kNucPenWords;
       for (int w = threadIdx.x; w < G::kChunk / 32; w += kThreads) out[w] = cm.bitmap[w];
@@ -1034,15 +1088,12 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
                                      flags, wp, cm);
   else if (lane() == 0) wp->flags = flags;
   if (NUC && rp.nucleus) {  // the row's range, and this chunk's count histogram
-    // the smallest finite register token (-inf slots count as +inf)
+    // the smallest finite register token (-inf slots are passed over)
     const TIn inf = (TIn)INFINITY;
     TIn lmn = inf;
     tk.new_pass();
 #pragma unroll
-    for (int e = 0; e < G::kEpt; e += 2) {
-      const TIn v0 = tk.rv(e), v1 = tk.rv(e + 1);
-      lmn = in_min3(lmn, v0 > -inf ? v0 : inf, v1 > -inf ? v1 : inf);
-    }
+    for (int e = 0; e < G::kEpt; e += 2) lmn = in_min3(lmn, finite_or_nan(tk.rv(e)), finite_or_nan(tk.rv(e + 1)));
     double zmn = (double)lmn;
     for (int i = 0; i < tk.np; ++i) {
       const double z = tk.pen_z(cm, i);
@@ -2917,6 +2968,24 @@ __global__ __launch_bounds__(kThreads) void k_nuc_window(SampleArgs a) {
 constexpr int kNucStage = 256;                   // tokens a wave stages before summing their mass
 constexpr int kNucCandWave = kCapChunk / kWaves;  // window tokens a wave stages
 
+// A token on its way from the registers to settle().
+template <typename TIn>
+struct NucStaged {
+  TIn z;
+  int idx;
+};
+
+// The smallest float whose bin (NucBin) is at least d: floor(zf * rz) - base >= d
+// exactly when zf >= (base + d) / rz, as scaling by a power of two is exact
+// (but for a product that underflows to -0, which counts as 0); bin 0 and
+// below hold every finite value, bins past the last none.
+__device__ __forceinline__ float nuc_edge(const NucRow& nr, int d) {
+  if (d <= 0) return -3.402823466e38f;
+  if (d >= kNucBins) return INFINITY;
+  const int q = nr.base + d;
+  return __double2float_ru((q == 0 ? -0x1p-150 : (double)q) / (double)nr.rz);
+}
+
 // The window's tokens go to the candidate slots (p and id); the tokens on
 // the row's smaller side of the window (nr.above) have their p summed per
 // segment.  Both are first staged per wave in LDS (a ballot per token step,
@@ -2926,7 +2995,7 @@ template <typename TIn, bool VEC>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) void k_nuc_cands(SampleArgs a) {
   using G = Geo<TIn>;
   __shared__ ChunkSmem cm;
-  __shared__ double stz[kWaves][kNucStage];
+  __shared__ NucStaged<TIn> stz[kWaves][kNucStage];
   __shared__ int over;
   const int C = a.ws.C;
   const int capc = a.ws.capc;
@@ -2947,55 +3016,61 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
     cm.cand_n = 0;
     over = 0;
   }
-  if (rp.pen_active) set_aside_penalised<TIn>(tk, nuc_pbits<TIn>(a, g), rp.pen, c0, cm);
+  if (rp.pen_active) set_aside_penalised<TIn>(tk, nuc_pbits<TIn>(a, g), rp.pen, c0, x, cm);
   wg_barrier();
   const YScale ys{rp.T, 1.0 / rp.T};
-  const NucBin nb(nr);
   const bool abv = nr.above != 0;
-  double* sz = stz[wave()];
+  NucStaged<TIn>* st = stz[wave()];
   StageRaw* cs = cm.sraw + wave() * kNucCandWave;
   uint32_t* cc = cm.scode + wave() * kNucCandWave;
   double acc = 0.0;  // this lane's share of the side's mass
-  int mn = 0, cn = 0;  // staged side tokens and window tokens (the same in every lane)
-  auto flush = [&]() {
-    for (int i = lane(); i < mn; i += kWave) acc += nuc_p(ys(sz[i]), nr, tab);
-    mn = 0;
+  int mn = 0, cn = 0;  // staged tokens and window tokens (the same in every lane)
+  // Per token: two compares, a ballot and a staged store, against 25
+  // instructions that formed the bin and staged the side and the window apart
+  // (1024 x 152 064: this kernel 204 -> 180 us, 13% of its tokens in range).
+  // The window and its smaller side are one range of z: [clo, cend) is the
+  // window, and the side goes on above it or below it.  -inf is in neither.
+  const float clo = nuc_edge(nr, nr.dlo), cend = nuc_edge(nr, nr.dhi + 1);
+  const float from = abv ? clo : -3.402823466e38f, to = abv ? INFINITY : cend;
+  // the tokens in range, 64 at a time: their p joins the side's mass or the
+  // window's list
+  auto settle = [&](bool on, double z, float zf, int idx) {
+    const double p = on ? nuc_p(ys(z), nr, tab) : 0.0;
+    const bool side = abv ? zf >= cend : zf < clo;
+    if (on && side) acc += p;
+    const uint64_t mc = __ballot(on && !side);
+    const int slot = mbcnt(mc, cn);
+    if (on && !side && slot < kNucCandWave) {
+      cs[slot].d = p;
+      cc[slot] = (uint32_t)idx;
+    }
+    cn += __popcll(mc);
   };
-  // the side's bins: above the window, or below it
-  const int slo = abv ? nr.dhi + 1 : 0;
-  const int shi = abv ? kNucBins - 1 : nr.dlo - 1;
-  // z: the token's (penalised) logit; zf: z rounded to float, which is
-  // what the bins see (exact for a register token).  A -inf token takes
-  // bin -1, outside both ranges; the tests are plain compares, no branches.
-  auto take = [&](double z, float zf, int idx) {
-    const int b = z > -INFINITY ? nb(zf) : -1;
-    const bool side = (b >= slo) & (b <= shi);
-    const bool cand = (b >= nr.dlo) & (b <= nr.dhi);
-    const uint64_t ms = __ballot(side);
-    if (ms != 0ull) {
-      if (side) sz[mbcnt(ms, mn)] = z;
-      mn += __popcll(ms);
-      if (mn > kNucStage - kWave) flush();
+  auto flush = [&]() {
+    for (int i0 = 0; i0 < mn; i0 += kWave) {
+      const int i = i0 + lane();
+      const NucStaged<TIn> s = st[min(i, mn - 1)];
+      settle(i < mn, (double)s.z, (float)s.z, s.idx);
     }
-    const uint64_t mc = __ballot(cand);
-    if (mc != 0ull) {
-      const int slot = mbcnt(mc, cn);
-      if (cand && slot < kNucCandWave) {
-        cs[slot].d = z;
-        cc[slot] = (uint32_t)idx;
-      }
-      cn += __popcll(mc);
-    }
+    mn = 0;
   };
   tk.new_pass();
 #pragma unroll
-  for (int e = 0; e < G::kEpt; ++e) take((double)tk.rv(e), (float)tk.rv(e), c0 + slot_q<TIn>(e));
+  for (int e = 0; e < G::kEpt; ++e) {
+    const float zf = (float)tk.rv(e);
+    const bool in = (zf >= from) & (zf < to);
+    const uint64_t m = __ballot(in);
+    if (in) st[mbcnt(m, mn)] = NucStaged<TIn>{tk.rv(e), c0 + slot_q<TIn>(e)};
+    mn += __popcll(m);
+    if (e % 2 == 1 && mn > kNucStage - 2 * kWave) flush();
+  }
+  flush();
   const int npmax = wave_max(tk.np);
   for (int i = 0; i < npmax; ++i) {
     const double z = i < tk.np ? tk.pen_z(cm, i) : -INFINITY;
-    take(z, (float)z, i < tk.np ? tk.pen_tok(cm, i) : 0);
+    const float zf = (float)z;
+    settle((zf >= from) & (zf < to), z, zf, i < tk.np ? tk.pen_tok(cm, i) : 0);
   }
-  flush();
   acc = wave_sum(acc);
   if (lane() == 0) a.ws.nexcl[(size_t)g * kWaves + wave()] = acc;
   // the staged window tokens: one reservation per wave, then to the slots
@@ -3008,7 +3083,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
     double* cz = a.ws.cz + (size_t)g * capc;
     int32_t* ci = a.ws.ci + (size_t)g * capc;
     for (int i = lane(); i < cn; i += kWave) {
-      cz[base + i] = nuc_p(ys(cs[i].d), nr, tab);
+      cz[base + i] = cs[i].d;
       ci[base + i] = (int)cc[i];
     }
   }
