@@ -205,11 +205,14 @@ int sample_impl(plh_ctx* c, const void* logits, int dtype, int64_t ld, int B, in
   a.nucleus_only = a.nucleus && (flags & PLH_SAMPLE_NUCLEUS_ONLY) ? 1 : 0;
   const bool f64 = dtype == PLH_F64;
   // the fast path gathers per-row state in LDS sized for V <= 262144
-  const bool small = V <= plh::kSmallV && !(flags & PLH_SAMPLE_ROWWISE);  // one launch, no workspace
+  // one launch, no workspace: rows of a small vocabulary, and ids of rows of
+  // a middling one
+  const bool small = V <= plh::kSmallV && !(flags & PLH_SAMPLE_ROWWISE);
+  const bool one = small || plh::one_launch_ids(B, V, c->num_cu);
   if (out_probs != nullptr || (flags & PLH_SAMPLE_ROWWISE) || V > kMaxVBitmap) {
     const bool probs = out_probs != nullptr && V <= plh::kProbsV && !(flags & PLH_SAMPLE_ROWWISE);
     const hipError_t e = small   ? plh::launch_sample_small(a, f64, c->stream, nullptr)
-                         : probs ? plh::launch_probs_rows(a, f64, c->stream)
+                         : probs ? plh::launch_probs_rows(a, f64, c->stream, nullptr)
                                  : plh::launch_sample_rows(a, f64, vec, c->stream);
     if (e != hipSuccess) return hip_fail(c, e, "plh_sample launch");
     return PLH_OK;
@@ -226,13 +229,14 @@ int sample_impl(plh_ctx* c, const void* logits, int dtype, int64_t ld, int B, in
     if (rc != PLH_OK) return rc;
     a.ws = plh::fast_ws_layout(c->scratch, B, V, f64);
     const hipError_t e = small ? plh::launch_sample_small(a, f64, c->stream, nullptr)
+                         : one ? plh::launch_probs_rows(a, f64, c->stream, nullptr)
                                : plh::launch_sample_fast(a, f64, vec, c->num_cu, c->stream, nullptr);
     if (e != hipSuccess) return hip_fail(c, e, "plh_sample_noalloc launch");
     c->scratch_stream = c->stream;
     c->scratch_open = true;
     return PLH_OK;
   }
-  if (!small) {
+  if (!one) {
     rc = reserve_ws(c, need);
     if (rc != PLH_OK) return rc;
     a.ws = plh::fast_ws_layout(c->ws, B, V, f64);
@@ -241,10 +245,11 @@ int sample_impl(plh_ctx* c, const void* logits, int dtype, int64_t ld, int B, in
   rc = timing_begin(c, ev);
   if (rc != PLH_OK) return rc;
   const hipError_t e = small ? plh::launch_sample_small(a, f64, c->stream, ev[1])
+                       : one ? plh::launch_probs_rows(a, f64, c->stream, ev[1])
                              : plh::launch_sample_fast(a, f64, vec, c->num_cu, c->stream, ev[1]);
   if (e != hipSuccess) return hip_fail(c, e, "plh_sample launch");
   if (c->timing) PLH_HIP(c, hipEventRecord(ev[2], c->stream), "hipEventRecord");
-  if (!small) {
+  if (!one) {
     c->ws_stream = c->stream;
     c->ws_open = true;
   }

@@ -152,12 +152,16 @@ struct HeadArgs {
 
 // Rows of at most kSmallV tokens: the whole call in one launch, no workspace.
 // `between` (when not null) is recorded after it.
-constexpr int kSmallV = 2048;
+constexpr int kSmallV = 1024;
 hipError_t launch_sample_small(const SampleArgs& a, bool f64, hipStream_t s, hipEvent_t between);
 // The processed distributions (and ids) of rows of kSmallV + 1 to kProbsV
 // tokens: one launch, no workspace.
 constexpr int kProbsV = 262144;
-hipError_t launch_probs_rows(const SampleArgs& a, bool f64, hipStream_t s);
+// The same for ids only (out_probs null): rows of up to kRowV tokens.
+constexpr int kRowV = 8192;
+bool one_launch_ids(int B, int V, int num_cu);
+// `between` (when not null) is recorded after the launch.
+hipError_t launch_probs_rows(const SampleArgs& a, bool f64, hipStream_t s, hipEvent_t between);
 hipError_t launch_sample_rows(const SampleArgs& a, bool f64, bool vec, hipStream_t s);
 // Fast path: workspace bytes for a [B, V] batch, its layout inside `base`
 // (256-byte aligned), and the two launches.

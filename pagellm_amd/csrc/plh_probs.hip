@@ -1,6 +1,6 @@
 // gfx950 kernel for the processed distributions of rows (probs(),
-// src/pagellm/engine/sampling.py:65-91, and the draw from them): one workgroup
-// of 1024 threads per row.
+// src/pagellm/engine/sampling.py:65-91), the draw from them, and the draw alone
+// for rows of a middling vocabulary: one workgroup of 1024 threads per row.
 //
 // The row's output is its scratch: once top-k is settled, one pass writes each
 // token's exp to its place in out_probs, and every later pass reads it back
@@ -199,15 +199,19 @@ __device__ __forceinline__ Cut select_key(const Each& each, uint64_t top, int sh
   }
 }
 
-template <typename TIn>
+// EXPORT: the row's distribution is wanted, and its place holds the exps.
+// Otherwise (ids only) they are held in LDS, and before them the penalised
+// logits, for rows of at most kRowV tokens.
+template <typename TIn, bool EXPORT>
 __global__ __launch_bounds__(kPT) void k_probs_row(SampleArgs a) {
   constexpr int kVW = 16 / (int)sizeof(TIn);
   typedef TIn VI __attribute__((ext_vector_type(kVW))) __attribute__((aligned(sizeof(TIn))));
   typedef double VO __attribute__((ext_vector_type(kVW))) __attribute__((aligned(8)));
   __shared__ ProbsSmem sm;
+  __shared__ alignas(16) double row_e[EXPORT ? 1 : kRowV];
   const int row = blockIdx.x, V = a.V, tid = threadIdx.x;
   const TIn* x = reinterpret_cast<const TIn*>(a.logits) + (int64_t)row * a.ld;
-  double* po = a.out_probs + (int64_t)row * V;
+  double* const po = EXPORT ? a.out_probs + (int64_t)row * V : nullptr;
   const RowParams rp = load_row_params(a, row);
   if (tid < 64) sm.exp_tab[tid] = kExp2Frac64[tid];
   if (rp.pen_active) {
@@ -264,16 +268,21 @@ __global__ __launch_bounds__(kPT) void k_probs_row(SampleArgs a) {
   };
   // the exps, once written
   auto pass_e = [&](auto f) {
-    pass([&](int t) { return *reinterpret_cast<const VO*>(po + t); }, [&](int t) { return po[t]; }, f);
+    if constexpr (EXPORT)
+      pass([&](int t) { return *reinterpret_cast<const VO*>(po + t); }, [&](int t) { return po[t]; }, f);
+    else
+      pass([&](int t) { return *reinterpret_cast<const VO*>(row_e + t); }, [&](int t) { return row_e[t]; }, f);
   };
   auto store = [&](int t, int n, const double (&p)[kVW]) {
     if (n == kVW) {
       VO v;
 #pragma unroll
       for (int e = 0; e < kVW; ++e) v[e] = p[e];
-      *reinterpret_cast<VO*>(po + t) = v;
+      if constexpr (EXPORT) *reinterpret_cast<VO*>(po + t) = v;
+      else *reinterpret_cast<VO*>(row_e + t) = v;
     } else if (n > 0) {
-      po[t] = p[0];
+      if constexpr (EXPORT) po[t] = p[0];
+      else row_e[t] = p[0];
     }
   };
 
@@ -283,17 +292,23 @@ __global__ __launch_bounds__(kPT) void k_probs_row(SampleArgs a) {
 #pragma unroll
     for (int e = 0; e < kVW; ++e)
       if (e < n) best = argmax_merge(best, ArgMax{z[e], t + e});
+    if constexpr (!EXPORT) store(t, n, z);  // the later passes over the logits
   });
+  auto pass_y = [&](auto f) {
+    if constexpr (EXPORT) pass_z(f);
+    else pass_e(f);
+  };
   best = wave_argmax(best);
   const double zmax = all_waves(best.v, sm.redd, [](double p, double q) { return p > q ? p : q; });
   if (rp.greedy) {  // :71-74
     const int id = min(all_waves(best.v == zmax ? best.i : INT_MAX, sm.redi, OpMin{}), V - 1);
+    if (tid == 0) a.out_ids[row] = id;
+    if constexpr (!EXPORT) return;
     typedef double V2 __attribute__((ext_vector_type(2))) __attribute__((aligned(8)));
     for (int i = 2 * tid; i < V; i += 2 * kPT) {  // a kilobyte per store of a wave
       if (i + 1 < V) *reinterpret_cast<V2*>(po + i) = V2{i == id ? 1.0 : 0.0, i + 1 == id ? 1.0 : 0.0};
       else po[i] = i == id ? 1.0 : 0.0;
     }
-    if (tid == 0) a.out_ids[row] = id;
     return;
   }
   const double T = rp.T, invT = 1.0 / T;
@@ -302,7 +317,7 @@ __global__ __launch_bounds__(kPT) void k_probs_row(SampleArgs a) {
   double z_lo = -INFINITY;
   if (rp.topk) {
     auto each = [&](auto fn) {
-      pass_z([&](int, int t, int n, double (&z)[kVW]) {
+      pass_y([&](int, int t, int n, double (&z)[kVW]) {
 #pragma unroll
         for (int e = 0; e < kVW; ++e)
           if (e < n) fn(key_of(z[e]), (uint64_t)1, t + e);
@@ -316,7 +331,7 @@ __global__ __launch_bounds__(kPT) void k_probs_row(SampleArgs a) {
   // ---- softmax over the survivors (:79-81): the exps to the row's output
   const PCalc pc{invT, zmax * invT, 1.0, z_lo, sm.exp_tab};
   double s = 0.0;
-  pass_z([&](int, int t, int n, double (&z)[kVW]) {
+  pass_y([&](int, int t, int n, double (&z)[kVW]) {
     double v[kVW];
 #pragma unroll
     for (int e = 0; e < kVW; ++e) {
@@ -412,7 +427,7 @@ __global__ __launch_bounds__(kPT) void k_probs_row(SampleArgs a) {
       uint64_t w[kVW], ts = 0;
 #pragma unroll
       for (int e = 0; e < kVW; ++e) {
-        w[e] = e < n ? to_fx(keep(po[t + e] * invS)) : 0;
+        w[e] = e < n ? to_fx(keep((EXPORT ? po[t + e] : row_e[t + e]) * invS)) : 0;
         ts += w[e];
       }
       uint64_t c = start + wave_scan_incl(ts, (uint64_t)0, OpAdd{}) - ts;
@@ -427,6 +442,7 @@ __global__ __launch_bounds__(kPT) void k_probs_row(SampleArgs a) {
     }
   }
 
+  if constexpr (!EXPORT) return;
   // ---- the distribution: top-p renormalises the kept mass (:89-90)
   pass_e([&](int, int t, int n, double (&d)[kVW]) {
     double p[kVW];
@@ -441,9 +457,23 @@ __global__ __launch_bounds__(kPT) void k_probs_row(SampleArgs a) {
 
 }  // namespace
 
-hipError_t launch_probs_rows(const SampleArgs& a, bool f64, hipStream_t s) {
-  if (f64) hipLaunchKernelGGL(k_probs_row<double>, dim3(a.B), dim3(kPT), 0, s, a);
-  else hipLaunchKernelGGL(k_probs_row<float>, dim3(a.B), dim3(kPT), 0, s, a);
+// Ids of rows of kSmallV + 1 to kRowV tokens.  Microseconds, the chunked path /
+// here, 16 rows: 4096 tokens top-k 20.1 / 13.2, top-p 49 / 12.8, top-k + top-p +
+// penalty 63 / 17.7, Zipf rows with top-p and penalty 27.8 / 12.6; 8192 tokens
+// 18.1 / 16.6, 53 / 16.6, 23.8 / 21.9, 27.4 / 15.6.  One workgroup fills a CU, so
+// past one row a CU the long rows with a top-k take longer (1024 x 8192: top-k
+// 56 / 64, top-k + top-p + penalty 73 / 88; 1024 x 4096: 62 / 49, 226 / 68).
+bool one_launch_ids(int B, int V, int num_cu) { return V <= kRowV / 2 || (V <= kRowV && B <= num_cu); }
+
+hipError_t launch_probs_rows(const SampleArgs& a, bool f64, hipStream_t s, hipEvent_t between) {
+  const bool e = a.out_probs != nullptr;
+  auto k = f64 ? (e ? k_probs_row<double, true> : k_probs_row<double, false>)
+               : (e ? k_probs_row<float, true> : k_probs_row<float, false>);
+  hipLaunchKernelGGL(k, dim3(a.B), dim3(kPT), 0, s, a);
+  if (between != nullptr) {
+    const hipError_t r = hipEventRecord(between, s);
+    if (r != hipSuccess) return r;
+  }
   return hipGetLastError();
 }
 

@@ -15,11 +15,10 @@
 // of a row padded to N = 2^n tokens.
 //
 // 16 rows, microseconds per call, the chunked path / here: 65 tokens 23.6 / 8.3
-// (top-k, top-p and penalty), 512 tokens 68 / 9.7, 2048 tokens top-k 20.1 / 16.9,
-// top-p 24.7 / 19.0, mixed 65 / 20; greedy rows 10.4 / 7.9.  At 4096 tokens the
-// sort costs more than the chunked path's second chain (28 / 39), so rows of
-// more than 2048 tokens stay there.  probs() of 16 rows: 65 tokens 66 / 8.4
-// against the general pipeline, 2048 tokens 62 / 21.
+// (top-k, top-p and penalty), 512 tokens 68 / 9.7, 1024 tokens 69 / 13.1; greedy
+// rows 10.5 / 8.  Past 1024 tokens the sort grows longer than the selection of
+// k_probs_row (2048 tokens: 20 here, 12.5 to 17.5 there).  probs() of 16 rows:
+// 65 tokens 66 / 8.4 against the general pipeline, 1000 tokens 67 / 13.5.
 #include "plh_device.h"
 #include "plh_fast.h"
 #include "plh_kernels.h"
@@ -279,14 +278,13 @@ __global__ __launch_bounds__(kThreads) void k_sample_small(SampleArgs a) {
   }
 }
 
-static_assert(kSmallV == 4 * kThreads, "the widest instantiation below");
+static_assert(kSmallV == 2 * kThreads, "the widest instantiation below");
 
 template <typename TIn>
 void launch_small_t(const SampleArgs& a, hipStream_t s) {
   const dim3 grid(a.B), block(kThreads);
   if (a.V <= kThreads) hipLaunchKernelGGL((k_sample_small<TIn, 1>), grid, block, 0, s, a);
-  else if (a.V <= 2 * kThreads) hipLaunchKernelGGL((k_sample_small<TIn, 2>), grid, block, 0, s, a);
-  else hipLaunchKernelGGL((k_sample_small<TIn, 4>), grid, block, 0, s, a);
+  else hipLaunchKernelGGL((k_sample_small<TIn, 2>), grid, block, 0, s, a);
 }
 
 }  // namespace

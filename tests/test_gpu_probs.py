@@ -46,7 +46,7 @@ def _rows(g, V, dtype):
 # first past the small kernel; a block of 1024 threads (float64: 2048 tokens,
 # float32: 4096) less one, whole and with one to three tokens past the last
 # 16-byte vector; more blocks than are loaded at once; an odd vocabulary
-@pytest.mark.parametrize("V", [2049, 4095, 4096, 4097, 8194, 16387, 32000, 50257])
+@pytest.mark.parametrize("V", [1025, 2049, 4095, 4096, 4097, 8192, 8194, 16387, 32000, 50257])
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
 def test_probs_rows(V, dtype):
     g = np.random.default_rng(V)
@@ -78,3 +78,8 @@ def test_probs_rows(V, dtype):
     w = dict(logits=x, params=params, contexts=hist, uniforms=u)
     mism, _ = compare_rows(w, [b for b in range(B) if not params[b].greedy], out.download(), f"probs V={V}")
     assert mism == 0
+    if V <= 8192:  # ids alone come from the same kernel, with the row in LDS
+        ids = c.empty((B,), np.int32)
+        c.sample(d["x"].ptr, _native.dtype_code(buf.dtype), V + 3, B, V, d["hi"].ptr, d["ho"].ptr, d["t"].ptr, d["k"].ptr,
+                 d["p"].ptr, d["r"].ptr, d["u"].ptr, ids.ptr, None, 0)
+        assert np.array_equal(ids.download(), out.download())
