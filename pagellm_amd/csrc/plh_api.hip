@@ -569,17 +569,24 @@ int plh_verify(plh_ctx* c, const void* p, const void* q, int dtype, int B, int k
   int rc = use_device(c);
   if (rc != PLH_OK) return rc;
   plh::VerifyArgs a{p, q, B, k, V, draft, accept_u, draw_u, draw_u_per_stop ? 1 : 0, out_tokens, out_n_acc};
-  rc = reserve_ws(c, plh::verify_ws_bytes(B, V));
-  if (rc != PLH_OK) return rc;
-  const plh::VerifyWs ws = plh::verify_ws_layout(c->ws, B, V);
+  const bool one = plh::verify_one_launch(B, V);
+  plh::VerifyWs ws{};
+  if (!one) {
+    rc = reserve_ws(c, plh::verify_ws_bytes(B, V));
+    if (rc != PLH_OK) return rc;
+    ws = plh::verify_ws_layout(c->ws, B, V);
+  }
   std::array<hipEvent_t, 3> ev{};
   rc = timing_begin(c, ev);
   if (rc != PLH_OK) return rc;
-  const hipError_t e = plh::launch_verify(a, ws, dtype == PLH_F64, c->stream, ev[1]);
+  const hipError_t e = one ? plh::launch_verify_row(a, dtype == PLH_F64, c->stream, ev[1])
+                           : plh::launch_verify(a, ws, dtype == PLH_F64, c->stream, ev[1]);
   if (e != hipSuccess) return hip_fail(c, e, "plh_verify launch");
   if (c->timing) PLH_HIP(c, hipEventRecord(ev[2], c->stream), "hipEventRecord");
-  c->ws_stream = c->stream;
-  c->ws_open = true;
+  if (!one) {
+    c->ws_stream = c->stream;
+    c->ws_open = true;
+  }
   return PLH_OK;
 }
 

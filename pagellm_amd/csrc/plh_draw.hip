@@ -24,48 +24,20 @@
 // float64 division per token; 512 x 152 064: 108 us, 5.8 TB/s.
 #include "plh_device.h"
 #include "plh_kernels.h"
+#include "plh_pieces.h"
 
 namespace plh {
 
 namespace {
 
-constexpr int kPiece = 512;         // tokens per piece
 constexpr int kDrawChunk = 32;   // pieces per workgroup of k_draw_parts
 constexpr int kMaxPieces = 2048;  // pieces whose sums k_draw_row holds (V <= 1 048 576)
 
-template <typename TIn>
-struct DrawGeo {
-  static constexpr int kVW = 16 / (int)sizeof(TIn);
-  static constexpr int kLoads = kPiece / (kVW * kWave);  // 16-byte loads per lane and piece
-  typedef TIn V __attribute__((ext_vector_type(kVW))) __attribute__((aligned(sizeof(TIn))));
-};
-
 __device__ __forceinline__ double weight_of(double v) { return v > 0.0 ? v : 0.0; }
 
-// The calling lane's tokens of piece s: load j holds tokens
-// s * 512 + (j * 64 + lane) * kVW onwards.  Tokens past the row weigh nothing.
 template <typename TIn>
-__device__ __forceinline__ void load_piece(const TIn* p, int V, int s, typename DrawGeo<TIn>::V (&x)[DrawGeo<TIn>::kLoads]) {
-  using G = DrawGeo<TIn>;
-  const int i0 = s * kPiece + lane() * G::kVW;
-  if (V - s * kPiece >= kPiece) {
-#pragma unroll
-    for (int j = 0; j < G::kLoads; ++j)
-      x[j] = *reinterpret_cast<const typename G::V*>(p + i0 + j * G::kVW * kWave);
-  } else {
-#pragma unroll
-    for (int j = 0; j < G::kLoads; ++j)
-#pragma unroll
-      for (int e = 0; e < G::kVW; ++e) {
-        const int i = i0 + j * G::kVW * kWave + e;
-        x[j][e] = i < V ? p[i] : TIn(0);
-      }
-  }
-}
-
-template <typename TIn>
-__device__ __forceinline__ double lane_sum(const typename DrawGeo<TIn>::V (&x)[DrawGeo<TIn>::kLoads]) {
-  using G = DrawGeo<TIn>;
+__device__ __forceinline__ double lane_sum(const typename PieceGeo<TIn>::V (&x)[PieceGeo<TIn>::kLoads]) {
+  using G = PieceGeo<TIn>;
   double t = 0.0;
 #pragma unroll
   for (int j = 0; j < G::kLoads; ++j)
@@ -79,7 +51,7 @@ __device__ __forceinline__ double lane_sum(const typename DrawGeo<TIn>::V (&x)[D
 // are dropped, so that no branch parts the loads.
 template <int U, typename TIn>
 __device__ __forceinline__ void sum_batch(const TIn* p, int s, int last, double* out) {
-  typename DrawGeo<TIn>::V x[U][DrawGeo<TIn>::kLoads];
+  typename PieceGeo<TIn>::V x[U][PieceGeo<TIn>::kLoads];
 #pragma unroll
   for (int i = 0; i < U; ++i) load_piece(p, INT_MAX, min(s + i, last), x[i]);
 #pragma unroll
@@ -92,7 +64,7 @@ __device__ __forceinline__ void sum_batch(const TIn* p, int s, int last, double*
 // Sums pieces s0 .. s1-1 of a row into out[0 ..], by one wave.
 template <typename TIn>
 __device__ __forceinline__ void sum_pieces(const TIn* p, int V, int s0, int s1, double* out) {
-  typename DrawGeo<TIn>::V tail[DrawGeo<TIn>::kLoads];
+  typename PieceGeo<TIn>::V tail[PieceGeo<TIn>::kLoads];
   const bool ragged = s0 < s1 && (int64_t)s1 * kPiece > V;  // the row's last piece, cut short
   const int last = ragged ? s1 - 2 : s1 - 1;
   if (ragged) load_piece(p, V, s1 - 1, tail);
@@ -111,68 +83,21 @@ __device__ __forceinline__ void sum_pieces(const TIn* p, int V, int s0, int s1, 
 // lane alike.
 template <typename TIn, class Sum>
 __device__ __forceinline__ int pick_token(const TIn* p, int V, double u, const Sum& sum, int n) {
-  using G = DrawGeo<TIn>;
-  double run = 0.0;
-  for (int base = 0; base < n; base += kWave)
-    run = lane_value(run + wave_scan_incl(sum(base + lane()), 0.0, OpAdd{}), kWave - 1);
-  const double W = run;
+  using G = PieceGeo<TIn>;
+  const double W = pieces_total(sum, n);
   // no mass, or more than a double holds, or u past the end: the last id
   // (sampling.py:98 clamps to V - 1)
   if (!(W > 0.0) || W > 1.7976931348623157e308 || u >= 1.0) return V - 1;
   const double t = fmax(u * W, 0.0);
-  // the first piece whose running total exceeds t, else the last with mass
-  int f = -1, last = -1;
-  double before = 0.0, blast = 0.0;
-  run = 0.0;
-  for (int base = 0; base < n && f < 0; base += kWave) {
-    const double v = sum(base + lane());
-    const double incl = run + wave_scan_incl(v, 0.0, OpAdd{});
-    const uint64_t pos = __ballot(v > 0.0), over = __ballot(v > 0.0 && incl > t);
-    if (over != 0) {
-      const int k = __builtin_ctzll(over);
-      f = base + k;
-      before = lane_value(incl - v, k);
-    } else if (pos != 0) {
-      const int k = 63 - __builtin_clzll(pos);
-      last = base + k;
-      blast = lane_value(incl - v, k);
-    }
-    run = lane_value(incl, kWave - 1);
-  }
-  const bool crossed = f >= 0;
-  if (!crossed) {
-    f = last;
-    before = blast;
-  }
+  const Crossing c = cross_pieces(sum, n, t);
   typename G::V x[G::kLoads];
-  load_piece(p, V, f, x);
-  int tok = -1, tail = -1;
+  load_piece(p, V, c.piece, x);
+  double w[G::kLoads][G::kVW];
 #pragma unroll
-  for (int j = 0; j < G::kLoads; ++j) {
-    double w[G::kVW], ts = 0.0;
+  for (int j = 0; j < G::kLoads; ++j)
 #pragma unroll
-    for (int e = 0; e < G::kVW; ++e) {
-      w[e] = weight_of((double)x[j][e]);
-      ts += w[e];
-    }
-    const double incl = wave_scan_incl(ts, 0.0, OpAdd{});
-    double cum = before + (incl - ts);
-    const int i0 = f * kPiece + (j * kWave + lane()) * G::kVW;
-    int hit = INT_MAX, pos = -1;
-#pragma unroll
-    for (int e = 0; e < G::kVW; ++e) {
-      cum += w[e];
-      if (w[e] > 0.0) {
-        pos = i0 + e;
-        if (hit == INT_MAX && cum > t) hit = i0 + e;
-      }
-    }
-    tail = max(tail, wave_max(pos));
-    const int h = wave_min(hit);
-    if (crossed && tok < 0 && h != INT_MAX) tok = h;
-    before += lane_value(incl, kWave - 1);
-  }
-  return tok >= 0 ? tok : tail;
+    for (int e = 0; e < G::kVW; ++e) w[j][e] = weight_of((double)x[j][e]);
+  return pick_in_piece<TIn>(c, t, w);
 }
 
 template <typename TIn>
@@ -196,7 +121,7 @@ __global__ __launch_bounds__(kThreads) void k_draw_row(DrawArgs a) {
       double mine = 0.0;
       const int first = i - lane();
       for (int k = 0; k < kWave && first + k < n; ++k) {
-        typename DrawGeo<TIn>::V x[DrawGeo<TIn>::kLoads];
+        typename PieceGeo<TIn>::V x[PieceGeo<TIn>::kLoads];
         load_piece(p, a.V, first + k, x);
         const double t = wave_sum(lane_sum<TIn>(x));
         if (lane() == k) mine = t;

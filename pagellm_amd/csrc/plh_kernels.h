@@ -175,6 +175,10 @@ hipError_t launch_sample_fast(const SampleArgs& a, bool f64, bool vec, int num_c
 size_t draw_ws_bytes(int B, int V, int num_cu);
 hipError_t launch_draw(const DrawArgs& a, bool f64, hipStream_t s);
 hipError_t launch_penalize(const PenalizeArgs& a, bool f64, hipStream_t s);
+// Verify in one launch (no workspace) where verify_one_launch says so; `between`
+// as below.
+bool verify_one_launch(int B, int V);
+hipError_t launch_verify_row(const VerifyArgs& a, bool f64, hipStream_t s, hipEvent_t between);
 // Verify: workspace bytes for B rows of V tokens, its layout, and the two
 // launches (stop positions and chunk sums, then the draw).
 size_t verify_ws_bytes(int B, int V);

@@ -8,8 +8,9 @@
 // acceptances the bonus row p_k; the emitted token is an inverse-CDF draw
 // over that row.
 //
-// A row's draw is spread over chunks of 4096 tokens, one workgroup each, so
-// that a batch of a few dozen rows still fills the chip:
+// Rows that one workgroup streams quickly take one launch (k_verify_row).  The
+// draw of a longer row is spread over chunks of 4096 tokens, one workgroup each,
+// so that a batch of a few dozen rows still fills the chip:
 //   k_verify_parts  (row, chunk)  stop position; float64 chunk sums of the
 //                                 residual and of p;
 //   k_verify_draw   (row)         W and the running chunk totals in one fixed
@@ -23,6 +24,7 @@
 // token of positive weight is taken (a neighbour of the boundary either
 // way).
 #include "plh_kernels.h"
+#include "plh_pieces.h"
 #include "plh_pipeline.h"
 
 namespace plh {
@@ -267,6 +269,134 @@ __global__ __launch_bounds__(kThreads) void k_verify_draw(VerifyArgs a, VerifyWs
   }
 }
 
+// The whole of a row in one launch: stop position, the piece sums (512 tokens)
+// of the residual and of p in LDS, and the draw from the crossing piece.
+// Bound by its chain for a few dozen rows: the accept tests' two gathers, one
+// CU's read of p and q (256 KB each at 32 000 float64), the piece read again.
+constexpr int kRowPieces = 128;  // V <= 65536
+
+// Piece sums of the residual and of p for pieces s .. s+U-1 (those past `last`
+// read as `last` and are dropped), all loads in flight together.
+template <int U, bool RES, typename TIn>
+__device__ __forceinline__ void verify_batch_sums(const TIn* p, const TIn* q, int s, int last, double* sr, double* sp) {
+  using G = PieceGeo<TIn>;
+  typename G::V x[U][G::kLoads], y[U][G::kLoads];
+#pragma unroll
+  for (int i = 0; i < U; ++i) {
+    load_piece(p, INT_MAX, min(s + i, last), x[i]);
+    if (RES) load_piece(q, INT_MAX, min(s + i, last), y[i]);
+  }
+#pragma unroll
+  for (int i = 0; i < U; ++i) {
+    double r = 0.0, w = 0.0;
+#pragma unroll
+    for (int j = 0; j < G::kLoads; ++j)
+#pragma unroll
+      for (int e = 0; e < G::kVW; ++e) {
+        w += draw_weight((double)x[i][j][e], 0.0, false, true);
+        if (RES) r += draw_weight((double)x[i][j][e], (double)y[i][j][e], true, true);
+      }
+    w = wave_sum(w);
+    if (RES) r = wave_sum(r);
+    if (lane() == 0 && s + i <= last) {
+      sp[s + i] = w;
+      sr[s + i] = r;
+    }
+  }
+}
+
+template <bool RES, typename TIn>
+__device__ __forceinline__ void verify_wave_sums(const TIn* p, const TIn* q, int V, double* sr, double* sp) {
+  using G = PieceGeo<TIn>;
+  const int n = (V - 1) / kPiece + 1, w = uniform(wave());
+  const int per = (n + kWaves - 1) / kWaves, s0 = min(w * per, n), s1 = min(s0 + per, n);
+  const bool ragged = s0 < s1 && s1 * kPiece > V;  // the row's last piece, cut short
+  const int last = ragged ? s1 - 2 : s1 - 1;
+  typename G::V x[G::kLoads], y[G::kLoads];
+  if (ragged) {
+    load_piece(p, V, s1 - 1, x);
+    if (RES) load_piece(q, V, s1 - 1, y);
+  }
+  int s = s0;
+  for (; s + 2 <= last; s += 4) verify_batch_sums<4, RES>(p, q, s, last, sr, sp);
+  if (s + 1 <= last) verify_batch_sums<2, RES>(p, q, s, last, sr, sp);
+  else if (s <= last) verify_batch_sums<1, RES>(p, q, s, last, sr, sp);
+  if (ragged) {
+    double r = 0.0, t = 0.0;
+#pragma unroll
+    for (int j = 0; j < G::kLoads; ++j)
+#pragma unroll
+      for (int e = 0; e < G::kVW; ++e) {
+        t += draw_weight((double)x[j][e], 0.0, false, true);
+        if (RES) r += draw_weight((double)x[j][e], (double)y[j][e], true, true);
+      }
+    t = wave_sum(t);
+    if (RES) r = wave_sum(r);
+    if (lane() == 0) {
+      sp[s1 - 1] = t;
+      sr[s1 - 1] = r;
+    }
+  }
+}
+
+template <typename TIn>
+__global__ __launch_bounds__(kThreads) void k_verify_row(VerifyArgs a) {
+  using G = PieceGeo<TIn>;
+  __shared__ double sr[kRowPieces], sp[kRowPieces];
+  const int b = blockIdx.x, k = a.k, V = a.V, n = (V - 1) / kPiece + 1;
+  const TIn* P = reinterpret_cast<const TIn*>(a.p) + (size_t)b * (k + 1) * V;
+  const TIn* Q = reinterpret_cast<const TIn*>(a.q) + (size_t)b * k * V;
+  int32_t* out = a.out_tokens + (size_t)b * (k + 1);
+  const int s = uniform(stop_position(a, P, Q, b));
+  if (s < 0) {
+    for (int i = threadIdx.x; i <= k; i += kThreads) out[i] = -1;
+    if (threadIdx.x == 0) a.out_n_acc[b] = -1;
+    return;
+  }
+  const TIn* ps = P + (size_t)s * V;
+  const TIn* qs = s < k ? Q + (size_t)s * V : ps;
+  const double u = a.draw_u[a.draw_u_per_stop ? (size_t)b * (k + 1) + s : (size_t)b];
+  if (s < k) verify_wave_sums<true>(ps, qs, V, sr, sp);
+  else verify_wave_sums<false>(ps, qs, V, sr, sp);
+  for (int i = threadIdx.x; i <= k; i += kThreads)
+    if (i != s) out[i] = i < s ? a.draft[(size_t)b * k + i] : -1;
+  wg_barrier();
+  if (wave() != 0) return;
+  const double wr = s < k ? pieces_total([&](int i) { return i < n ? sr[i] : 0.0; }, n) : 0.0;
+  const bool resid = wr > 0.0;  // speculative.py:55-58
+  const double* part = resid ? sr : sp;
+  auto sum = [&](int i) { return i < n ? part[i] : 0.0; };
+  const double W = resid ? wr : pieces_total(sum, n);
+  int tok = V - 1;  // sampling.py:98: no mass takes the last id
+  if (W > 0.0) {
+    const double t = u * W;
+    const Crossing c = cross_pieces(sum, n, t);
+    if (c.piece >= 0) {
+      typename G::V x[G::kLoads], y[G::kLoads];
+      load_piece(ps, V, c.piece, x);
+      load_piece(qs, V, c.piece, y);
+      double w[G::kLoads][G::kVW];
+#pragma unroll
+      for (int j = 0; j < G::kLoads; ++j)
+#pragma unroll
+        for (int e = 0; e < G::kVW; ++e) w[j][e] = draw_weight((double)x[j][e], (double)y[j][e], resid, true);
+      const int f = pick_in_piece<TIn>(c, t, w);
+      if (f >= 0) tok = f;
+    }
+  }
+  if (lane() == 0) {
+    out[s] = tok;
+    a.out_n_acc[b] = s;
+  }
+}
+
+// One launch for rows one workgroup streams in the time of a second launch, two
+// for longer ones.  Microseconds, k = 4, two launches / one: float64 64 x 4096
+// 11.0 / 8.9, 64 x 32 000 11.8 / 10.2, 256 x 32 000 25.6 / 20.4, 8 x 50 257 10.8 /
+// 11.3, 64 x 50 257 15.9 / 14.5, 8 x 128 256 10.8 / 22.6, 64 x 128 256 24.4 / 29.5;
+// float32 64 x 32 000 12.3 / 8.6, 64 x 50 257 14.6 / 11.0, 64 x 128 256 21.9 / 23.3.
+bool verify_one_launch(int B, int V) { return V <= 40000 || (V <= kRowPieces * kPiece && B > 16); }
+
 namespace {
 size_t up256(size_t v) { return (v + 255) / 256 * 256; }
 }  // namespace
@@ -297,6 +427,16 @@ hipError_t launch_verify_t(const VerifyArgs& a, const VerifyWs& ws, hipStream_t 
     if (e != hipSuccess) return e;
   }
   hipLaunchKernelGGL((k_verify_draw<TIn>), dim3(a.B), block, 0, s, a, ws);
+  return hipGetLastError();
+}
+
+hipError_t launch_verify_row(const VerifyArgs& a, bool f64, hipStream_t s, hipEvent_t between) {
+  if (f64) hipLaunchKernelGGL(k_verify_row<double>, dim3(a.B), dim3(kThreads), 0, s, a);
+  else hipLaunchKernelGGL(k_verify_row<float>, dim3(a.B), dim3(kThreads), 0, s, a);
+  if (between != nullptr) {
+    const hipError_t e = hipEventRecord(between, s);
+    if (e != hipSuccess) return e;
+  }
   return hipGetLastError();
 }
 

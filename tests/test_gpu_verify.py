@@ -241,3 +241,32 @@ def test_random_verify_batches(seed):
         for b in np.nonzero((n != rn) | (toks != rt).any(1))[0]:
             gap = verify_boundary_gap(p64[b], q64[b], list(draft[b]), au[b], float(ru[b]))
             assert gap < DRAW_GAP, (it, int(b), toks[b].tolist(), rt[b].tolist(), gap)
+
+
+# around the 512-token pieces and the waves' shares of them, and the sizes at
+# which one launch gives way to two (40 000 for few rows, 65 536 for more)
+@pytest.mark.parametrize("B,V", [(3, 511), (3, 512), (3, 513), (3, 4609), (3, 40000), (3, 40001), (17, 65536),
+                                 (17, 65537)])
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+def test_verify_piece_and_launch_edges(B, V, dtype):
+    """Residual and bonus draws with spread mass, with mass in single tokens at
+    the pieces' ends, and with an all-zero residual (p drawn instead)."""
+    g = np.random.default_rng(V)
+    k = 2
+    p, q = g.random((B, k + 1, V)).astype(dtype), g.random((B, k, V)).astype(dtype)
+    ends = np.unique(np.minimum([0, 511, 512, V // 2, V - 1], V - 1))
+    p[1] = 0
+    p[1, :, ends] = 1
+    q[1] = 0.5 * p[1, :k]
+    q[2] = p[2, :k]  # identical: p / q = 1, rejected only by u = 1 - 2^-53 not below 1; the bonus row is drawn
+    draft = g.integers(0, V, (B, k))
+    draft[1] = ends[-1]
+    au, ru = g.random((B, k)), g.random(B)
+    au[0] = 1 - 2.0 ** -53  # rejected unless p >= q at the draft token
+    toks, n = verify_batch(p, q, draft, au, ru)
+    p64, q64 = p.astype(np.float64), q.astype(np.float64)
+    rt, rn = oracle.verify_batch(p64, q64, draft, au, ru)
+    assert np.array_equal(n, rn)
+    for b in range(B):
+        if not np.array_equal(toks[b], rt[b]):
+            assert verify_boundary_gap(p64[b], q64[b], list(draft[b]), au[b], ru[b]) < 1e-12, b
