@@ -17,6 +17,7 @@ here raises.
 
 from __future__ import annotations
 
+import struct
 from typing import Sequence
 
 import numpy as np
@@ -50,10 +51,23 @@ def _as_float_rows(x) -> np.ndarray:
     return np.ascontiguousarray(a)
 
 
+def _int64_row(context) -> np.ndarray:
+    """``np.asarray(context, dtype=np.int64).reshape(-1)``.  A list or tuple of
+    integers (what the engine keeps, ``llm_engine.py:283``) goes through
+    ``struct.pack``, a third of numpy's time per element; anything else, and
+    anything struct refuses, goes to numpy."""
+    if type(context) is list or type(context) is tuple:
+        try:
+            return np.frombuffer(struct.pack(f"{len(context)}q", *context), dtype=np.int64)
+        except struct.error:
+            pass
+    return np.asarray(context, dtype=np.int64).reshape(-1)
+
+
 def _history_ids(context, V: int) -> np.ndarray:
     """Token ids of one history as int32 in [0, V): numpy indexing semantics
     (negative ids wrap, ids outside [-V, V) raise IndexError)."""
-    ids = np.asarray(context, dtype=np.int64).reshape(-1)
+    ids = _int64_row(context)
     if ids.size:
         lo, hi = int(ids.min()), int(ids.max())
         if hi >= V or lo < -V:
@@ -74,15 +88,19 @@ def _pack_histories(contexts, params: Sequence[SamplingParams], B: int, V: int):
         return None, None
     if len(contexts) != B:
         raise ValueError(f"expected {B} contexts, got {len(contexts)}")
-    parts, off = [], np.zeros(B + 1, dtype=np.int64)
+    parts, sizes = [], [0] * (B + 1)
     for b in range(B):
         ctx = contexts[b]
-        n = 0
         if ctx is not None and params[b].repetition_penalty != 1.0 and len(ctx) > 0:
-            ids = _history_ids(ctx, V)
+            ids = _int64_row(ctx)
             parts.append(ids)
-            n = ids.size
-        off[b + 1] = off[b] + n
+            sizes[b + 1] = ids.size
+    off = np.cumsum(sizes, dtype=np.int64)
+    ids = np.concatenate(parts) if parts else np.zeros(0, dtype=np.int64)
+    # one range check for all rows; with an id outside [0, V), row by row (the
+    # first bad row raises, negative ids wrap)
+    if ids.size and (int(ids.min()) < 0 or int(ids.max()) >= V):
+        ids = np.concatenate([_history_ids(part, V) for part in parts])
     if off[-1] == 0:
         return None, None
     if V > MAX_PENALTY_VOCAB:
@@ -91,7 +109,7 @@ def _pack_histories(contexts, params: Sequence[SamplingParams], B: int, V: int):
             "the kernels mark a row's penalised tokens in an on-chip bitmap of that many bits; "
             "the reference (sampling.py:52-62) has no such limit"
         )
-    return np.concatenate(parts), off
+    return ids.astype(np.int32, copy=False), off
 
 
 def _pack_params(params: Sequence[SamplingParams]):

@@ -155,3 +155,29 @@ def test_penalised_rows_beyond_the_bitmap_fail_on_the_host_with_the_reason():
     assert _pack_histories([[]], [pen], 1, V) == (None, None)
     ids, off = _pack_histories([[1, 2, 3]], [pen], 1, MAX_PENALTY_VOCAB)
     assert list(ids) == [1, 2, 3] and list(off) == [0, 3]
+
+
+def test_pack_histories_takes_what_numpy_takes():
+    """Lists and tuples of ints are packed with struct; the other forms, and
+    the errors, are numpy's: each against np.asarray(context, int64) row by
+    row, with numpy's indexing semantics."""
+    from pagellm_amd.sampling import SamplingParams, _pack_histories
+
+    on, off = SamplingParams(repetition_penalty=1.1), SamplingParams()
+    V = 50
+    forms = [[1, 2, 3], (4, 4, 49), np.array([5, 6]), np.array([7], np.int32), range(3), [np.int64(8), True], [-1, 0],
+             [1.0, 2.9], [[1, 2], [3, 4]], [], None, np.zeros(0, np.int64)]
+    for ctxs in ([f] for f in forms):
+        ids, o = _pack_histories(ctxs, [on], 1, V)
+        want = np.asarray(ctxs[0] if ctxs[0] is not None else [], dtype=np.int64).reshape(-1) % V
+        if want.size == 0:
+            assert ids is None and o is None
+        else:
+            assert ids.dtype == np.int32 and np.array_equal(ids, want) and o.tolist() == [0, want.size]
+    ids, o = _pack_histories([[1, 2], [3], [-2]], [on, off, on], 3, V)
+    assert ids.tolist() == [1, 2, 48] and o.tolist() == [0, 2, 2, 3]
+    for bad, err in (([[1], [50], [-51]], IndexError), ([[2 ** 63]], OverflowError), ([["x"]], ValueError)):
+        with pytest.raises(err) as e:
+            _pack_histories(bad, [on] * len(bad), len(bad), V)
+        if err is IndexError:
+            assert "index 50" in str(e.value)  # the first bad row
