@@ -596,7 +596,7 @@ HeadPlan head_plan(int N, int D, int V, int64_t ldw, int num_cu) {
   HeadPlan best{lo, 1};
   double best_us = plan_us(best, N, D, V, num_cu);
   for (int rows = lo; rows <= hi; rows *= 2)
-    for (int slices = 1; slices <= 32; slices *= 2) {
+    for (int slices = 1; slices <= (N <= 4096 ? 32 : 1); slices *= 2) {  // k_head_sum's grid holds N in y
       const HeadPlan p{rows, slices};
       const double us = plan_us(p, N, D, V, num_cu);
       if (us < best_us) {

@@ -30,7 +30,6 @@
 //   k_sample_rows    the general pipeline for every row (and the only kernel
 //                    that exports the processed distribution, probs()).
 // Others:
-//   k_draw           inverse-CDF draw from given distributions (draw()).
 //   k_penalize       repetition penalty on a copy (apply_repetition_penalty()).
 #include "plh_fast.h"
 #include "plh_kernels.h"

@@ -37,6 +37,7 @@ def _case(seed, N, D, V, scale=1.0):
     (256, 128, 4096),    # full row tile, V on the vector-load path
     (17, 4096, 300),     # deep k loop
     (5, 1, 7),           # one column of k
+    (4097, 520, 65),     # more rows than are ever summed over slices of k
 ])
 def test_head_matches_oracle(N, D, V):
     print(f"[head] N={N} D={D} V={V}", flush=True)
