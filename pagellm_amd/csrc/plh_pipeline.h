@@ -4,8 +4,7 @@
 // temperature -> top-k -> softmax -> top-p -> inverse-CDF draw, greedy
 // argmax) over a logits row streamed from HBM once per pass, 32 consecutive
 // tokens per thread per group with all of a group's loads in flight
-// together.  It is the general path (any parameters, any distribution) and
-// the path that exports the processed distribution.  Sorting is replaced by
+// together.  It is the general path (any parameters, any distribution).  Sorting is replaced by
 // selection: top-k is an MSD radix select by count on order-preserving
 // 64-bit keys of the penalised logits; the top-p cut is an MSD radix select
 // by fixed-point probability mass on the same keys (p is non-decreasing in

@@ -27,8 +27,9 @@
 //                    decide exactly is finished by the general pipeline in
 //                    the same workgroup.
 // General path:
-//   k_sample_rows    the general pipeline for every row (and the only kernel
-//                    that exports the processed distribution, probs()).
+//   k_sample_rows    the general pipeline for every row (plh_small.hip and
+//                    plh_probs.hip hold the one-launch kernels for shorter
+//                    rows and for probs()).
 // Others:
 //   k_penalize       repetition penalty on a copy (apply_repetition_penalty()).
 #include "plh_fast.h"
