@@ -53,13 +53,16 @@ def _as_float_rows(x) -> np.ndarray:
 
 def _int64_row(context) -> np.ndarray:
     """``np.asarray(context, dtype=np.int64).reshape(-1)``.  A list or tuple of
-    integers (what the engine keeps, ``llm_engine.py:283``) goes through
-    ``struct.pack``, a third of numpy's time per element; anything else, and
-    anything struct refuses, goes to numpy."""
-    if type(context) is list or type(context) is tuple:
+    Python ints (what the engine keeps, ``llm_engine.py:283``) goes through
+    ``struct.pack``, which converts a list whose ints are in the CPU's caches in
+    a third of numpy's time (fetching them dominates otherwise).  Everything
+    else is numpy's to convert or to refuse, also an element further on that
+    struct does not take or whose ``__index__`` raises (a float tensor, an array
+    of one element)."""
+    if (type(context) is list or type(context) is tuple) and len(context) > 0 and type(context[0]) is int:
         try:
             return np.frombuffer(struct.pack(f"{len(context)}q", *context), dtype=np.int64)
-        except struct.error:
+        except Exception:
             pass
     return np.asarray(context, dtype=np.int64).reshape(-1)
 

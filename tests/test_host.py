@@ -181,3 +181,25 @@ def test_pack_histories_takes_what_numpy_takes():
             _pack_histories(bad, [on] * len(bad), len(bad), V)
         if err is IndexError:
             assert "index 50" in str(e.value)  # the first bad row
+
+
+@pytest.mark.parametrize("wrap", [list, tuple])
+def test_history_elements_that_are_not_integers_for_struct(wrap):
+    """Elements with an ``__index__`` that raises (float tensors, arrays of one
+    element) are numpy's to convert, at the front of a history or further on."""
+    import torch
+
+    class OnlyInt:
+        def __int__(self):
+            return 5
+
+        def __index__(self):
+            raise ValueError("no index")
+
+    on = SamplingParams(repetition_penalty=1.1)
+    for el in (torch.tensor(3.0), torch.tensor([3]), np.array([3]), np.array(3.0), np.array([[3]]), OnlyInt(), 3.7):
+        forms = [[el], [el, el]] + ([[1, 2, el]] if np.ndim(el) == 0 else [])
+        for f in forms:
+            want = np.asarray(f, dtype=np.int64).reshape(-1)
+            ids, o = S._pack_histories([wrap(f)], [on], 1, 50)
+            assert ids.tolist() == want.tolist() and o.tolist() == [0, want.size], f
