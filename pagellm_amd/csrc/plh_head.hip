@@ -290,7 +290,12 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
 // stage ahead on its own made every stage wait for the other's newest loads
 // (4096 x 128 256: 64 rows 690 us, 256 rows 1 420 us).  The stage loop has no
 // branch and no predicated load for the same reason: at a join the loads'
-// registers were copied, which waits for them.
+// registers were copied, which waits for them.  Nor does it lean on a range
+// check, which covers the lanes' offsets of a buffer load but not its scalar
+// offset: every address is clamped into W (a last row or column read twice
+// instead), and act is 0 for k >= D, up to whole units of 4 stages.  (A
+// descriptor per row of W, exact in its range, costs 40 scalar instructions
+// a stage: 4096 x 128 256, 256 rows 1 240 -> 1 320 us, 64 rows 460 -> 520 us.)
 // Inputs that the split cannot carry (infinities, float32 overflow on the
 // way, results so small that bf16 parts underflow) show up in the result;
 // the wave then forms its tile again on the fp32 matrix cores.
@@ -305,9 +310,11 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kSplitCols = 256;  // columns per workgroup
 constexpr int kSplitK = 16;      // k per stage: one MFMA step
-constexpr int kSplitMaxLdw = 1 << 24;  // a stage's rows of W lie within 2^30 bytes
+constexpr int kSplitMaxLdw = 1 << 24;  // a thread's eight rows of W lie within 2^29 bytes
 
 __host__ __device__ constexpr int split_stages(int D) { return (D + kSplitK - 1) / kSplitK; }
+// k groups of act: whole units of the 4 stages that a thread holds at most
+__host__ __device__ constexpr int split_groups(int D) { return (split_stages(D) + 3) / 4 * 8; }
 
 struct Split8 {
   u32x4 part[3];  // hi, mid, lo: 8 bf16 each
@@ -339,7 +346,7 @@ __global__ __launch_bounds__(kThreads) void k_head_prep_split(HeadArgs a) {
   const int n = blockIdx.x, D = a.D;
   const float* x = a.h + (size_t)n * a.ldh;
   const float r = row_rinv(a, x);
-  const int groups = 2 * split_stages(D);
+  const int groups = split_groups(D);
   u32x4* o = static_cast<u32x4*>(a.act);
   for (int kg = threadIdx.x; kg < groups; kg += kThreads) {
     float v[8];
@@ -365,7 +372,7 @@ __device__ __forceinline__ bool split_suspect(float x) {
 // its first part, a NaN in the first two)
 __device__ __forceinline__ float split_act(const HeadArgs& a, int n, int k) {
   const uint16_t* act = static_cast<const uint16_t*>(a.act);
-  const int groups = 2 * split_stages(a.D);
+  const int groups = split_groups(a.D);
   float part[3];
 #pragma unroll
   for (int p = 0; p < 3; ++p)
@@ -417,24 +424,22 @@ k_head_split(HeadArgs a) {
   const int rt = (int)a.lda / BM;
   const int v0 = (int)(blockIdx.x / rt) * kSplitCols, n0 = (int)(blockIdx.x % rt) * BM;
   const int wr = w % G::kWR, wc = w / G::kWR;
-  // this slice's stages, a multiple of kPF (the last slice's stages past nk
-  // multiply W by 0)
-  const int nk = split_stages(D), groups = 2 * nk, units = (nk + kPF - 1) / kPF;
+  // this slice's stages, a multiple of kPF
+  const int groups = split_groups(D), units = (split_stages(D) + kPF - 1) / kPF;
   const int sb = (int)((int64_t)units * blockIdx.z / gridDim.z) * kPF;
   const int se = (int)((int64_t)units * (blockIdx.z + 1) / gridDim.z) * kPF;
 
   // W: this thread's column and k group (uniform over the wave); act: 16-byte
   // pieces tid, tid + 512, ... of the stage's 6 BM
   const int col = (int)threadIdx.x & (kSplitCols - 1), kg = w >> 2;
-  const int pitch = (int)a.ldw * 4;
+  const int pitch = (int)a.ldw * 4, voff = min(col, V - 1 - v0) * 4;
   float wreg[kPF][8];
   u32x4 areg[kPF][G::kA];
   auto load = [&](int s, float (&o)[8], u32x4 (&x)[G::kA]) {
-    const int rows = min(D - s * kSplitK, kSplitK);  // rows past D, and stages past the slice's, read as 0
-    const int bytes = s < se && rows > 0 ? (rows - 1) * pitch + (V - v0) * 4 : 0;
+    const int k0 = min(s * kSplitK + kg * 8, D - 1), last = min(D - 1 - k0, 7) * pitch;
     const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<float*>(a.w + (size_t)s * kSplitK * a.ldw + v0), (short)0, bytes, 0x00020000);
-    const u32x4* ap = static_cast<const u32x4*>(a.act) + (size_t)(2 * min(s, nk - 1)) * a.lda + n0;
+        const_cast<float*>(a.w + (size_t)k0 * a.ldw + v0), (short)0, 0x7fffffff, 0x00020000);
+    const u32x4* ap = static_cast<const u32x4*>(a.act) + (size_t)min(2 * s, groups - 2) * a.lda + n0;
 #pragma unroll
     for (int i = 0; i < G::kA; ++i) {
       const int q = min((int)threadIdx.x + kThreads * i, 6 * BM - 1);
@@ -442,7 +447,7 @@ k_head_split(HeadArgs a) {
     }
 #pragma unroll
     for (int j = 0; j < 8; ++j)
-      o[j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, col * 4, (kg * 8 + j) * pitch, 0));
+      o[j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, voff, min(j * pitch, last), 0));
   };
   auto store = [&](int buf, const float (&o)[8], const u32x4 (&x)[G::kA]) {
     const Split8 s = split8(o);
@@ -609,7 +614,7 @@ HeadPlan head_plan(int N, int D, int V, int64_t ldw, int num_cu) {
 
 size_t act_bytes(const HeadPlan& p, int N, int D) {
   const size_t rows = ((size_t)N + p.rows - 1) / p.rows * p.rows;
-  return (size_t)split_stages(D) * kSplitK * rows * (p.rows <= 32 ? 4 : 6);
+  return (size_t)split_groups(D) * 8 * rows * (p.rows <= 32 ? 4 : 6);
 }
 
 size_t head_ws_bytes(int N, int D, int V, int64_t ldw, int num_cu) {

@@ -114,6 +114,35 @@ def test_values_at_the_ends_of_float32(N, D, V):
     assert np.all(err <= TOL * bound[ok][:, rest] + 1e-30)
 
 
+@pytest.mark.parametrize("N,D,V", [
+    (40, 72, 70001),      # 64-row tile, k and columns ragged
+    (40, 1000, 333),      # ... in slices of k
+    (100, 1016, 70001),   # 128-row tile
+    (200, 1000, 128255),  # 256-row tile
+])
+def test_nothing_past_the_end_of_lm_head_is_read(N, D, V):
+    """What lies behind the matrix in memory (here: rows of the same
+    allocation) changes no bit of the logits.  A value read there would meet a
+    zero of act, but for NaN and infinities, after which the element is formed
+    again in another order."""
+    import torch
+
+    print(f"[head] tail N={N} D={D} V={V}", flush=True)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(D)
+    buf = torch.randn((D + 48, V), generator=g, device="cuda")
+    buf[:D] *= 0.02
+    W = buf[:D]
+    norm = 1 + 0.1 * torch.randn(D, generator=g, device="cuda")
+    h = torch.randn((N, D), generator=g, device="cuda")
+    ref = None
+    for tail in (0.0, float("nan"), float("inf"), 3e38):
+        buf[D:] = tail
+        got = H.rms_norm_lm_head(h, norm, W, 1e-5)
+        ref = got.clone() if ref is None else ref
+        assert torch.equal(got, ref), tail
+
+
 def test_tiny_rows_and_eps():
     """Rows of norm ~1e-3 (eps visible), an all-zero row (r = 1/sqrt(eps))."""
     h, norm, W = _case(3, 6, 96, 257, scale=1e-3)
