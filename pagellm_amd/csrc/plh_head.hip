@@ -269,7 +269,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
 // ------------------------------------------------------------ many rows
 //
 // float32 products on the bf16 matrix cores.  A float32 x is exactly
-// hi + mid + lo, three bf16 values (its 24 significant bits, 8 at a time), so
+// hi + mid + lo, three bf16 values (its 24 significant bits, 8 at a time; both
+// operands are first scaled by 2^47, so that the parts of the smallest float32,
+// 2^-149, are normal bf16 numbers), so
 //   a * w = ah*wh + (ah*wm + am*wh) + (ah*wl + am*wm + al*wh) + rest,
 // with |rest| <= 2^-22 |a w| (three products of 2^-8 * 2^-16 and below), each
 // product exact and summed in float32 by v_mfma_f32_32x32x16_bf16.  Six bf16
@@ -296,9 +298,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
 // instead), and act is 0 for k >= D, up to whole units of 4 stages.  (A
 // descriptor per row of W, exact in its range, costs 40 scalar instructions
 // a stage: 4096 x 128 256, 256 rows 1 240 -> 1 320 us, 64 rows 460 -> 520 us.)
-// Inputs that the split cannot carry (infinities, float32 overflow on the
-// way, results so small that bf16 parts underflow) show up in the result;
-// the wave then forms its tile again on the fp32 matrix cores.
+// What the parts cannot carry leaves no finite sum (infinities, operands of
+// 2^81 on, sums that reach 2^34 on the way); those 32 x 32 tiles are formed again
+// on the fp32 matrix cores, from the rows in float32.
 //
 // Against the fp32 matrix product in 256-row tiles, 4096 x 128 256: 256 rows
 // 2 020 -> 1 230 us (1.31 PFLOP/s of bf16 products, the rate of a large bf16
@@ -311,6 +313,8 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 constexpr int kSplitCols = 256;  // columns per workgroup
 constexpr int kSplitK = 16;      // k per stage: one MFMA step
 constexpr int kSplitMaxLdw = 1 << 24;  // a thread's eight rows of W lie within 2^29 bytes
+constexpr int kRedoK = 32;       // k per step of the float32 product
+constexpr float kSplitScale = 0x1p47f, kSplitUnscale = 0x1p-94f;
 
 __host__ __device__ constexpr int split_stages(int D) { return (D + kSplitK - 1) / kSplitK; }
 // k groups of act: whole units of the 4 stages that a thread holds at most
@@ -320,12 +324,12 @@ struct Split8 {
   u32x4 part[3];  // hi, mid, lo: 8 bf16 each
 };
 
-// x = hi + mid + lo by truncation: each remainder is exact.
+// 2^47 x = hi + mid + lo by truncation: each remainder is exact.
 __device__ __forceinline__ Split8 split8(const float (&x)[8]) {
   Split8 s;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    float a = x[2 * i], b = x[2 * i + 1];
+    float a = x[2 * i] * kSplitScale, b = x[2 * i + 1] * kSplitScale;
 #pragma unroll
     for (int p = 0; p < 3; ++p) {
       const uint32_t ua = __float_as_uint(a), ub = __float_as_uint(b);
@@ -340,14 +344,18 @@ __device__ __forceinline__ Split8 split8(const float (&x)[8]) {
 }
 
 // act for k_head_split: part p, k group kg (8 k), row n at
-// ((p * groups + kg) * lda + n) * 8; zero for k >= D (rows N .. lda-1 are not
-// written: an accumulator row depends on its own act row only).
+// ((p * groups + kg) * lda + n) * 8; zero for k >= D and for the rows N .. lda-1
+// that fill the last tile.  Also each row in float32 (act32, zero for k >= D).
 __global__ __launch_bounds__(kThreads) void k_head_prep_split(HeadArgs a) {
   const int n = blockIdx.x, D = a.D;
-  const float* x = a.h + (size_t)n * a.ldh;
-  const float r = row_rinv(a, x);
   const int groups = split_groups(D);
   u32x4* o = static_cast<u32x4*>(a.act);
+  if (n >= a.N) {
+    for (int i = threadIdx.x; i < 3 * groups; i += kThreads) o[(size_t)i * a.lda + n] = u32x4{0u, 0u, 0u, 0u};
+    return;
+  }
+  const float* x = a.h + (size_t)n * a.ldh;
+  const float r = row_rinv(a, x);
   for (int kg = threadIdx.x; kg < groups; kg += kThreads) {
     float v[8];
 #pragma unroll
@@ -355,44 +363,42 @@ __global__ __launch_bounds__(kThreads) void k_head_prep_split(HeadArgs a) {
       const int d = 8 * kg + e;
       v[e] = d < D ? (x[d] * r) * a.norm[d] : 0.0f;
     }
+    f32x4* row = reinterpret_cast<f32x4*>(a.act32 + ((size_t)n * groups + kg) * 8);
+    row[0] = f32x4{v[0], v[1], v[2], v[3]};
+    row[1] = f32x4{v[4], v[5], v[6], v[7]};
     const Split8 s = split8(v);
 #pragma unroll
     for (int p = 0; p < 3; ++p) o[((size_t)p * groups + kg) * a.lda + n] = s.part[p];
   }
 }
 
-// A sum that the bf16 parts may not carry: not finite, or below 2^-80 without
-// being 0.
-__device__ __forceinline__ bool split_suspect(float x) {
-  const float y = fabsf(x);
-  return !(y <= 3.4028234663852886e38f) || (y < 8.2718061255302767e-25f && y > 0.0f);
-}
+__device__ __forceinline__ bool not_finite(float x) { return !(fabsf(x) <= 3.4028234663852886e38f); }
 
-// act[n][k] in float32, from its parts (exact; a non-finite value is all in
-// its first part, a NaN in the first two)
-__device__ __forceinline__ float split_act(const HeadArgs& a, int n, int k) {
-  const uint16_t* act = static_cast<const uint16_t*>(a.act);
-  const int groups = split_groups(a.D);
-  float part[3];
-#pragma unroll
-  for (int p = 0; p < 3; ++p)
-    part[p] = __uint_as_float((uint32_t)act[(((size_t)p * groups + (k >> 3)) * a.lda + n) * 8 + (k & 7)] << 16);
-  return part[1] != part[1] ? (part[0] == part[0] ? part[0] : part[1]) : part[0] + (part[1] + part[2]);
-}
-
-// One 32 x 32 tile of out, rows n.. and columns v.., on the fp32 matrix cores.
+// One 32 x 32 tile of out, rows n.. and columns v.., on the fp32 matrix cores:
+// half-wave h takes k 4h .. 4h+3 of every eight.
 __device__ __forceinline__ f32x16 head_tile_f32(const HeadArgs& a, int n, int v) {
-  const int l = lane(), D = a.D;
-  const int row = n + (l & 31), col = min(v + (l & 31), a.V - 1);
+  constexpr int kStep = kRedoK / 8;
+  const int l = lane(), D = a.D, half = 4 * (l >> 5);
+  const int row = min(n + (l & 31), a.N - 1), col = min(v + (l & 31), a.V - 1);
+  const float* x = a.act32 + (size_t)row * split_groups(D) * 8 + half;
   f32x16 acc;
 #pragma unroll
   for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
-#pragma unroll 8
-  for (int k0 = 0; k0 < D; k0 += 2) {
-    const int k = k0 + (l >> 5), kc = min(k, D - 1);
-    const float x = split_act(a, row, kc);
-    const float y = a.w[(size_t)kc * a.ldw + col];
-    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(k < D ? x : 0.0f, k < D ? y : 0.0f, acc, 0, 0, 0);
+  for (int kb = 0; kb < D; kb += kRedoK, x += kRedoK) {
+    const int k0 = kb + half;
+    f32x4 xs[kStep];
+    float ys[kStep][4];
+#pragma unroll
+    for (int i = 0; i < kStep; ++i) {
+      xs[i] = *reinterpret_cast<const f32x4*>(x + 8 * i);
+#pragma unroll
+      for (int t = 0; t < 4; ++t) ys[i][t] = a.w[(size_t)min(k0 + 8 * i + t, D - 1) * a.ldw + col];
+    }
+#pragma unroll
+    for (int i = 0; i < kStep; ++i)
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(xs[i][t], k0 + 8 * i + t < D ? ys[i][t] : 0.0f, acc, 0, 0, 0);
   }
   return acc;
 }
@@ -504,31 +510,35 @@ k_head_split(HeadArgs a) {
   // accumulator r of lane l holds row 8*(r/4) + 4*(l/32) + r%4, column l%32
   const int nb = n0 + wr * 64 + 4 * (l >> 5), vb = v0 + c0;
   auto row_of = [&](int mt, int r) { return nb + 32 * mt + 8 * (r >> 2) + (r & 3); };
-  bool redo = false;
-  if (gridDim.z == 1) {  // slices are checked where they are summed
-#pragma unroll
-    for (int mt = 0; mt < 2; ++mt)
-#pragma unroll
-      for (int nt = 0; nt < kNT; ++nt)
-#pragma unroll
-        for (int r = 0; r < 16; ++r)
-          if (split_suspect(acc[mt][nt][r])) redo = redo || (row_of(mt, r) < a.N && vb + 32 * nt < V);
-  }
-  const bool f32 = __ballot(redo) != 0;
   const HeadOut to = head_out(a);
+  const float scale = gridDim.z == 1 ? kSplitUnscale : 1.0f;  // slices: where they are added up
 #pragma unroll
   for (int mt = 0; mt < 2; ++mt)
 #pragma unroll
-    for (int nt = 0; nt < kNT; ++nt) {
-      const int v = vb + 32 * nt;
-      f32x16 y = acc[mt][nt];
-      if (f32) y = head_tile_f32(a, n0 + wr * 64 + 32 * mt, v0 + wc * 32 * kNT + 32 * nt);
+    for (int nt = 0; nt < kNT; ++nt)
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        const int n = row_of(mt, r);
-        if (n < a.N && v < V) to.p[(size_t)n * to.ld + v] = y[r];
+        const int n = row_of(mt, r), v = vb + 32 * nt;
+        if (n < a.N && v < V) to.p[(size_t)n * to.ld + v] = acc[mt][nt][r] * scale;
       }
+  if (gridDim.z > 1) return;
+  uint32_t redo = 0;  // bit 2 nt + mt: that tile of this wave
+#pragma unroll
+  for (int nt = 0; nt < kNT; ++nt)
+#pragma unroll
+    for (int mt = 0; mt < 2; ++mt) {
+      bool bad = false;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) bad |= not_finite(acc[mt][nt][r]);
+      if (__ballot(bad) != 0) redo |= 1u << (2 * nt + mt);
     }
+  for (; redo != 0; redo &= redo - 1) {
+    const int mt = __builtin_ctz(redo) & 1, nt = __builtin_ctz(redo) >> 1, v = vb + 32 * nt;
+    const f32x16 y = head_tile_f32(a, n0 + wr * 64 + 32 * mt, v0 + wc * 32 * kNT + 32 * nt);
+#pragma unroll
+    for (int r = 0; r < 16; ++r)
+      if (row_of(mt, r) < a.N && v < V) to.p[(size_t)row_of(mt, r) * to.ld + v] = y[r];
+  }
 }
 
 // ------------------------------------------------------------ slices of k
@@ -545,10 +555,13 @@ __global__ __launch_bounds__(256) void k_head_sum(HeadArgs a, int slices) {
 #pragma unroll 8
   for (int z = 0; z < slices; ++z) s += p[z * pitch];
   if constexpr (SPLIT) {
-    if (split_suspect(s)) {
+    if (not_finite(s)) {
+      const float* x = a.act32 + (size_t)n * split_groups(a.D) * 8;
       s = 0.0f;
 #pragma unroll 8
-      for (int k = 0; k < a.D; ++k) s = fmaf(split_act(a, n, k), a.w[(size_t)k * a.ldw + v], s);
+      for (int k = 0; k < a.D; ++k) s = fmaf(x[k], a.w[(size_t)k * a.ldw + v], s);
+    } else {
+      s *= kSplitUnscale;
     }
   }
   a.out[(size_t)n * a.ldo + v] = s;
@@ -612,14 +625,30 @@ HeadPlan head_plan(int N, int D, int V, int64_t ldw, int num_cu) {
   return best;
 }
 
-size_t act_bytes(const HeadPlan& p, int N, int D) {
-  const size_t rows = ((size_t)N + p.rows - 1) / p.rows * p.rows;
-  return (size_t)split_groups(D) * 8 * rows * (p.rows <= 32 ? 4 : 6);
+// The workspace: act in the product's layout, for k_head_split also in float32;
+// the partial sums.  Offsets in bytes.
+struct HeadWs {
+  size_t act32, part, bytes;
+};
+
+HeadWs head_ws(const HeadPlan& p, int N, int D, int V) {
+  const size_t rows = ((size_t)N + p.rows - 1) / p.rows * p.rows, K = (size_t)split_groups(D) * 8;
+  const bool split = p.rows > 32;
+  size_t at = K * rows * (split ? 6 : 4);
+  auto take = [&](size_t bytes) {
+    const size_t o = (at + 255) / 256 * 256;
+    at = o + bytes;
+    return o;
+  };
+  HeadWs w{};
+  w.act32 = take(split ? K * N * sizeof(float) : 0);
+  w.part = take(p.slices > 1 ? (size_t)p.slices * N * V * sizeof(float) : 0);
+  w.bytes = at;
+  return w;
 }
 
 size_t head_ws_bytes(int N, int D, int V, int64_t ldw, int num_cu) {
-  const HeadPlan p = head_plan(N, D, V, ldw, num_cu);
-  return act_bytes(p, N, D) + 256 + (p.slices > 1 ? (size_t)p.slices * N * V * sizeof(float) : 0);
+  return head_ws(head_plan(N, D, V, ldw, num_cu), N, D, V).bytes;
 }
 
 template <int R>
@@ -634,14 +663,17 @@ template <int BM>
 void launch_split(HeadArgs a, int slices, hipStream_t s) {
   const unsigned rt = (unsigned)((a.N + BM - 1) / BM);
   a.lda = (int64_t)rt * BM;
-  hipLaunchKernelGGL(k_head_prep_split, dim3(a.N), dim3(kThreads), 0, s, a);
+  hipLaunchKernelGGL(k_head_prep_split, dim3((unsigned)a.lda), dim3(kThreads), 0, s, a);
   hipLaunchKernelGGL(k_head_split<BM>, dim3((unsigned)((a.V + kSplitCols - 1) / kSplitCols) * rt, 1, (unsigned)slices),
                      dim3(kThreads), 0, s, a);
 }
 
 hipError_t launch_head(HeadArgs a, int num_cu, hipStream_t s) {
   const HeadPlan p = head_plan(a.N, a.D, a.V, a.ldw, num_cu);
-  a.part = reinterpret_cast<float*>(static_cast<char*>(a.act) + (act_bytes(p, a.N, a.D) + 255) / 256 * 256);
+  const HeadWs ws = head_ws(p, a.N, a.D, a.V);
+  char* base = static_cast<char*>(a.act);
+  a.act32 = reinterpret_cast<float*>(base + ws.act32);
+  a.part = reinterpret_cast<float*>(base + ws.part);
   a.lda = (int64_t)((a.N + p.rows - 1) / p.rows) * p.rows;
   switch (p.rows) {
     case 16: launch_skinny<16>(a, p.slices, s); break;

@@ -146,6 +146,7 @@ struct HeadArgs {
   int64_t ldo;
   void* act;          // workspace: the normalised rows in the product's operand layout
   int64_t lda;        // rows of act (whole row tiles)
+  float* act32;       // workspace [N, D padded to whole stages]: the rows in float32 (k_head_split)
   float* part;        // workspace [slices, N, V]: partial sums, with several slices of k
   int N, D, V;
 };

@@ -143,6 +143,33 @@ def test_nothing_past_the_end_of_lm_head_is_read(N, D, V):
         assert torch.equal(got, ref), tail
 
 
+@pytest.mark.parametrize("N,D,V", [(8, 64, 1000), (40, 64, 70000), (40, 512, 300)])  # few rows; one slice, several
+@pytest.mark.parametrize("small", ["weights", "rows", "neither"])
+def test_small_operands_against_large_ones(N, D, V, small):
+    """Operands whose low bits (or all of them) lie below bf16's range, with
+    ordinary logits: the other operand is large; and logits of 2^40.  Limit: a float32 sum in any
+    order is within D * 2^-24 of the bound, and each factor of act adds a
+    rounding or two (TOL covers both)."""
+    print(f"[head] small {small} N={N} D={D} V={V}", flush=True)
+    h, norm, W = _case(23, N, D, V)
+    if small == "weights":
+        norm *= np.float32(2.0 ** 64)
+        W = W * np.float32(2.0 ** -60)  # ordinary columns of such a matrix
+        for c, t in enumerate((124, 112, 104, 140, 126, 118)):
+            W[:, 3 + 40 * c] = (50 * W[:, 3 + 40 * c].astype(np.float64) * 2.0 ** (60 - t)).astype(np.float32)
+    elif small == "neither":
+        norm *= np.float32(2.0 ** 42)
+    else:
+        norm *= np.float32(2.0 ** -124)
+        W = W * np.float32(2.0 ** 64)
+    a = oracle.rms_norm(h, norm, np.float32(1e-5)).astype(np.float64)
+    ref, bound = a @ W.astype(np.float64), np.abs(a) @ np.abs(W.astype(np.float64))
+    got = H.rms_norm_lm_head(h, norm, W, 1e-5)
+    # act is rounded to float32's subnormal step, and so is each product
+    step = 2.0 ** -149 * (np.abs(W.astype(np.float64)).sum(0) + D) if small == "rows" else D * 2.0 ** -149
+    assert np.all(np.abs(got - ref) <= TOL * bound + step), float(np.max(np.abs(got - ref) / (bound + step)))
+
+
 def test_tiny_rows_and_eps():
     """Rows of norm ~1e-3 (eps visible), an all-zero row (r = 1/sqrt(eps))."""
     h, norm, W = _case(3, 6, 96, 257, scale=1e-3)
