@@ -269,17 +269,25 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
 // ------------------------------------------------------------ many rows
 //
 // float32 products on the bf16 matrix cores.  A float32 x is exactly
-// hi + mid + lo, three bf16 values (its 24 significant bits, 8 at a time; both
-// operands are first scaled by 2^47, so that the parts of the smallest float32,
-// 2^-149, are normal bf16 numbers), so
+// hi + mid + lo, three bf16 values (both operands are first scaled by 2^47, so
+// that the parts of the smallest float32, 2^-149, are normal bf16 numbers), so
 //   a * w = ah*wh + (ah*wm + am*wh) + (ah*wl + am*wm + al*wh) + rest,
-// with |rest| <= 2^-22 |a w| (three products of 2^-8 * 2^-16 and below), each
-// product exact and summed in float32 by v_mfma_f32_32x32x16_bf16.  Six bf16
-// products cost 6/16 of one on the fp32 matrix cores (2.5 PFLOP/s against 157
-// TFLOP/s), and a sum over k is rounded 6 times per 16 k instead of 8.
-// Against float64 the result is no further off than the fp32 matrix product
-// (2-norm, N(0, 1) rows, 0.02 N(0, 1) weights): 1.02e-6 against 1.1e-6 at
-// D = 4096, 4.9e-7 against 5.6e-7 at 1000, less with several slices of k.
+// each product exact and summed in float32 by v_mfma_f32_32x32x16_bf16.  With
+// parts rounded to nearest |rest| <= 1.01 * 2^-24 of the operands' powers of two
+// (am*wl and al*wm, 2^-8 * 2^-17 each), of either sign: half the last bit of a
+// float32 product.  (Truncated parts are 2^-7 and 2^-15 and all of x's sign: rest
+// was up to 2^-21 and one-sided, and sums of like signs dropped their low
+// products on the way, 1.2e-5 of the sum at D = 4096.)  Six bf16 products cost
+// 6/16 of one on the fp32 matrix cores (2.5 PFLOP/s against 157 TFLOP/s), and a
+// sum over k is rounded 6 times per 16 k instead of 8.  2-norm error against
+// float64 in units of 2^-24, the fp32 matrix product / here (one slice):
+//   D                          1     2     4     8    64   256   1000   4096
+//   N(0,1) x 0.02 N(0,1)    0.42  0.56  0.65  0.84  2.35  4.77   9.55  19.2
+//                           0.61  0.58  0.54  0.52  1.77  3.94   8.16  16.8
+//   U(1,2) x U(1,2)         0.45  0.51  0.60  0.75  2.03  3.88   7.79  15.9
+//                           0.60  0.48  0.48  0.50  1.41  2.89   5.30   9.9
+// and less with several slices of k.  Sums of fewer than kSplitMinD products take
+// the fp32 kernel.
 //
 // k_head_split<BM>: a BM-row x 256-column tile per workgroup, 8 waves of 64
 // rows x (BM / 2) columns (at least 32), k in stages of 16.  act comes split
@@ -303,16 +311,19 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
 // on the fp32 matrix cores, from the rows in float32.
 //
 // Against the fp32 matrix product in 256-row tiles, 4096 x 128 256: 256 rows
-// 2 020 -> 1 230 us (1.31 PFLOP/s of bf16 products, the rate of a large bf16
-// matrix product here), 128 rows 2 000 -> 740 us, 64 rows 2 000 -> 590 us, bound
-// by W's way through a CU; 45 x 1000 x 50 257: 293 -> 61 us.
+// 2 010 -> 1 220-1 270 us (1.27-1.33 PFLOP/s of bf16 products, the rate of a large
+// bf16 matrix product here), 128 rows 2 005 -> 735-770 us, 64 rows 2 000 -> 470-485
+// us, bound by W's way through a CU; 45 x 1000 x 50 257: 290 -> 55-57 us.
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kSplitCols = 256;  // columns per workgroup
 constexpr int kSplitK = 16;      // k per stage: one MFMA step
 constexpr int kSplitMaxLdw = 1 << 24;  // a thread's eight rows of W lie within 2^29 bytes
+constexpr int kSplitMinD = 4;    // products a sum has at least
 constexpr int kRedoK = 32;       // k per step of the float32 product
 constexpr float kSplitScale = 0x1p47f, kSplitUnscale = 0x1p-94f;
 
@@ -324,19 +335,21 @@ struct Split8 {
   u32x4 part[3];  // hi, mid, lo: 8 bf16 each
 };
 
-// 2^47 x = hi + mid + lo by truncation: each remainder is exact.
+// 2^47 x = hi + mid + lo, each the bf16 nearest to what is left: each remainder
+// is exact, and the last a bf16 itself (|mid| <= 2^-8 and |lo| <= 2^-17 of the
+// power of two below x, both signs).
 __device__ __forceinline__ Split8 split8(const float (&x)[8]) {
   Split8 s;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    float a = x[2 * i] * kSplitScale, b = x[2 * i + 1] * kSplitScale;
+    f32x2 r{x[2 * i] * kSplitScale, x[2 * i + 1] * kSplitScale};
 #pragma unroll
     for (int p = 0; p < 3; ++p) {
-      const uint32_t ua = __float_as_uint(a), ub = __float_as_uint(b);
-      s.part[p][i] = __builtin_amdgcn_perm(ub, ua, 0x07060302u);  // the upper halves of b and a
+      const uint32_t u = __builtin_bit_cast(uint32_t, __builtin_convertvector(r, bf16x2));
+      s.part[p][i] = u;
       if (p < 2) {
-        a -= __uint_as_float(ua & 0xffff0000u);
-        b -= __uint_as_float(ub & 0xffff0000u);
+        r[0] -= __uint_as_float(u << 16);
+        r[1] -= __uint_as_float(u & 0xffff0000u);
       }
     }
   }
@@ -503,6 +516,13 @@ k_head_split(HeadArgs a) {
                                                                   0, 0, 0);
       }
       store(buf ^ 1, wreg[(i + 1) % kPF], areg[(i + 1) % kPF]);
+      // the split's 60 vector instructions among the products, not behind them
+      // (64 rows x 4096 x 128 256: 505 -> 483 us, 45 x 1000 x 50 257: 64 -> 57 us)
+#pragma unroll
+      for (int q = 0; q < 12 * kNT; ++q) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                             // an MFMA ...
+        __builtin_amdgcn_sched_group_barrier(0x002, (60 + 12 * kNT) / (12 * kNT), 0);  // ... and its share
+      }
       wg_barrier();
     }
   }
@@ -609,7 +629,7 @@ double plan_us(const HeadPlan& p, int N, int D, int V, int num_cu) {
 // of 16, 410 us in one of 32).  Slices fill the chip where the columns alone
 // do not (4096 x 1000, 8 rows: 44 us in one slice, 15 us in 16).
 HeadPlan head_plan(int N, int D, int V, int64_t ldw, int num_cu) {
-  const bool skinny = N <= 32 || ldw > kSplitMaxLdw;
+  const bool skinny = N <= 32 || (D < kSplitMinD && N <= 65535 * 32) || ldw > kSplitMaxLdw;  // row tiles: the grid's y
   const int lo = skinny ? (N <= 16 ? 16 : 32) : 64, hi = skinny ? lo : 256;
   HeadPlan best{lo, 1};
   double best_us = plan_us(best, N, D, V, num_cu);

@@ -170,6 +170,26 @@ def test_small_operands_against_large_ones(N, D, V, small):
     assert np.all(np.abs(got - ref) <= TOL * bound + step), float(np.max(np.abs(got - ref) / (bound + step)))
 
 
+@pytest.mark.parametrize("N,D,V", [(40, 1, 4096), (40, 2, 4096), (40, 3, 4096), (40, 4, 4096), (40, 8, 4096),
+                                   (40, 64, 60000), (40, 1000, 333), (200, 1000, 50257), (256, 4096, 60000)])
+def test_sums_of_like_signs(N, D, V):
+    """Sums of D products in U(1, 4), where no error cancels: the 2-norm error
+    against float64 is within that of D float32 additions, whose roundings
+    (uniform, 2^-24 / sqrt(3) of the running sum) give 2^-24 sqrt(D) / 3, or one
+    last bit of the result for short sums."""
+    import torch
+
+    print(f"[head] like signs N={N} D={D} V={V}", flush=True)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(D)
+    W = 1 + torch.rand((D, V), generator=g, device="cuda")
+    a = 1 + torch.rand(D, generator=g, device="cuda")
+    got = H.rms_norm_lm_head(torch.ones((N, D), device="cuda"), a, W, 0.0).double()  # r = 1: act is a
+    ref = a.double() @ W.double()
+    err = float((got - ref).norm() / ref.norm() / N ** 0.5)
+    assert err <= 2.0 ** -24 * max(1.0, D ** 0.5 / 3), err * 2 ** 24
+
+
 def test_tiny_rows_and_eps():
     """Rows of norm ~1e-3 (eps visible), an all-zero row (r = 1/sqrt(eps))."""
     h, norm, W = _case(3, 6, 96, 257, scale=1e-3)
