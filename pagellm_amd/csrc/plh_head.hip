@@ -133,11 +133,14 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
   // half of the waves' accumulators at a time
   __shared__ f32x4 sm[kWaves / 2][S::kCG * kRegs][64];
   const int D = a.D, V = a.V, l = lane(), w = uniform(wave());
-  const int v0 = ANY ? (int)blockIdx.x * kSkinnyCols : min((int)blockIdx.x * kSkinnyCols, V - kSkinnyCols);
+  // the row tiles of one column tile side by side (more than one: rows of W far
+  // apart, or short sums)
+  const int rt = (a.N + R - 1) / R, tile = (int)(blockIdx.x % (unsigned)rt);
+  const int vx = (int)(blockIdx.x / (unsigned)rt) * kSkinnyCols, v0 = ANY ? vx : min(vx, V - kSkinnyCols);
   const int c = l % R, q = l / R;
-  const int n0 = blockIdx.y * R;
+  const int n0 = tile * R;
   const float* act =
-      static_cast<const float*>(a.act) + (size_t)blockIdx.y * skinny_groups(D, R) * S::kG * R + (size_t)(q * R + c) * 4;
+      static_cast<const float*>(a.act) + (size_t)tile * skinny_groups(D, R) * S::kG * R + (size_t)(q * R + c) * 4;
 
   typename A::T acc[S::kCG][4];
 #pragma unroll
@@ -629,7 +632,7 @@ double plan_us(const HeadPlan& p, int N, int D, int V, int num_cu) {
 // of 16, 410 us in one of 32).  Slices fill the chip where the columns alone
 // do not (4096 x 1000, 8 rows: 44 us in one slice, 15 us in 16).
 HeadPlan head_plan(int N, int D, int V, int64_t ldw, int num_cu) {
-  const bool skinny = N <= 32 || (D < kSplitMinD && N <= 65535 * 32) || ldw > kSplitMaxLdw;  // row tiles: the grid's y
+  const bool skinny = N <= 32 || D < kSplitMinD || ldw > kSplitMaxLdw;
   const int lo = skinny ? (N <= 16 ? 16 : 32) : 64, hi = skinny ? lo : 256;
   HeadPlan best{lo, 1};
   double best_us = plan_us(best, N, D, V, num_cu);
@@ -674,7 +677,7 @@ size_t head_ws_bytes(int N, int D, int V, int64_t ldw, int num_cu) {
 template <int R>
 void launch_skinny(const HeadArgs& a, int slices, hipStream_t s) {
   hipLaunchKernelGGL(k_head_prep<R>, dim3(a.N), dim3(kThreads), 0, s, a);
-  const dim3 grid((unsigned)((a.V + kSkinnyCols - 1) / kSkinnyCols), (unsigned)((a.N + R - 1) / R), (unsigned)slices);
+  const dim3 grid((unsigned)((a.V + kSkinnyCols - 1) / kSkinnyCols) * (unsigned)((a.N + R - 1) / R), 1, (unsigned)slices);
   if (a.V < kSkinnyCols || a.ldw > kSplitMaxLdw) hipLaunchKernelGGL((k_head_skinny<R, true>), grid, dim3(kThreads), 0, s, a);
   else hipLaunchKernelGGL((k_head_skinny<R, false>), grid, dim3(kThreads), 0, s, a);
 }

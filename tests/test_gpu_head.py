@@ -190,6 +190,23 @@ def test_sums_of_like_signs(N, D, V):
     assert err <= 2.0 ** -24 * max(1.0, D ** 0.5 / 3), err * 2 ** 24
 
 
+@pytest.mark.parametrize("N,V,ldw", [(2_100_000, 3, 3), (2_100_000, 3, (1 << 24) + 4), (70, 200, (1 << 24) + 4)])
+def test_many_rows_and_rows_of_lm_head_far_apart(N, V, ldw):
+    """The few-rows kernel over many row tiles: short sums, and rows of W that
+    lie more than 64 MB apart (r, act and the sums: at most 8 roundings of 2^-24)."""
+    import torch
+
+    print(f"[head] N={N} V={V} ldw={ldw}", flush=True)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(V)
+    W = torch.randn((2, ldw), generator=g, device="cuda")[:, :V]
+    h = torch.randn((N, 2), generator=g, device="cuda")
+    norm = torch.tensor([1.5, -0.5], device="cuda")
+    got = H.rms_norm_lm_head(h, norm, W, 1e-5).double()
+    a = h.double() * torch.rsqrt((h.double() ** 2).mean(1, keepdim=True) + 1e-5) * norm.double()
+    assert bool(((got - a @ W.double()).abs() <= 1e-6 * (a.abs() @ W.double().abs())).all())
+
+
 def test_tiny_rows_and_eps():
     """Rows of norm ~1e-3 (eps visible), an all-zero row (r = 1/sqrt(eps))."""
     h, norm, W = _case(3, 6, 96, 257, scale=1e-3)
