@@ -311,7 +311,11 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
 // a stage: 4096 x 128 256, 256 rows 1 240 -> 1 320 us, 64 rows 460 -> 520 us.)
 // What the parts cannot carry leaves no finite sum (infinities, operands of
 // 2^81 on, sums that reach 2^34 on the way); those 32 x 32 tiles are formed again
-// on the fp32 matrix cores, from the rows in float32.
+// on the fp32 matrix cores, from the rows in float32.  Not for a row of act that
+// holds a NaN: its sums are NaN already, and one broken request in a batch would
+// have every column tile formed again (256 x 4096 x 128 256: 3 010 us against
+// 1 220).  What is left of that is broken weights: an infinite lm_head value 1 450 us,
+// an infinite norm value 5 100 us.
 //
 // Against the fp32 matrix product in 256-row tiles, 4096 x 128 256: 256 rows
 // 2 010 -> 1 220-1 270 us (1.27-1.33 PFLOP/s of bf16 products, the rate of a large
@@ -361,23 +365,28 @@ __device__ __forceinline__ Split8 split8(const float (&x)[8]) {
 
 // act for k_head_split: part p, k group kg (8 k), row n at
 // ((p * groups + kg) * lda + n) * 8; zero for k >= D and for the rows N .. lda-1
-// that fill the last tile.  Also each row in float32 (act32, zero for k >= D).
+// that fill the last tile.  Also each row in float32 (act32, zero for k >= D), and
+// whether it holds a NaN (the rows past N count as such).
 __global__ __launch_bounds__(kThreads) void k_head_prep_split(HeadArgs a) {
   const int n = blockIdx.x, D = a.D;
   const int groups = split_groups(D);
   u32x4* o = static_cast<u32x4*>(a.act);
   if (n >= a.N) {
     for (int i = threadIdx.x; i < 3 * groups; i += kThreads) o[(size_t)i * a.lda + n] = u32x4{0u, 0u, 0u, 0u};
+    if (threadIdx.x == 0) a.nan_rows[n] = 1;
     return;
   }
   const float* x = a.h + (size_t)n * a.ldh;
   const float r = row_rinv(a, x);
+  __shared__ int red[kWaves];
+  int nan = 0;
   for (int kg = threadIdx.x; kg < groups; kg += kThreads) {
     float v[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
       const int d = 8 * kg + e;
       v[e] = d < D ? (x[d] * r) * a.norm[d] : 0.0f;
+      nan |= v[e] != v[e];
     }
     f32x4* row = reinterpret_cast<f32x4*>(a.act32 + ((size_t)n * groups + kg) * 8);
     row[0] = f32x4{v[0], v[1], v[2], v[3]};
@@ -386,6 +395,8 @@ __global__ __launch_bounds__(kThreads) void k_head_prep_split(HeadArgs a) {
 #pragma unroll
     for (int p = 0; p < 3; ++p) o[((size_t)p * groups + kg) * a.lda + n] = s.part[p];
   }
+  nan = block_max(nan, red);
+  if (threadIdx.x == 0) a.nan_rows[n] = nan;
 }
 
 __device__ __forceinline__ bool not_finite(float x) { return !(fabsf(x) <= 3.4028234663852886e38f); }
@@ -553,7 +564,12 @@ k_head_split(HeadArgs a) {
       bool bad = false;
 #pragma unroll
       for (int r = 0; r < 16; ++r) bad |= not_finite(acc[mt][nt][r]);
-      if (__ballot(bad) != 0) redo |= 1u << (2 * nt + mt);
+      if (__ballot(bad) == 0) continue;
+      uint32_t left = 0;  // bit r: not finite, and its row holds no NaN
+#pragma unroll
+      for (int r = 0; r < 16; ++r) left |= not_finite(acc[mt][nt][r]) ? 1u << r : 0u;
+      for (int r = 0; r < 16; ++r) left &= ~((uint32_t)a.nan_rows[row_of(mt, r)] << r);
+      if (__ballot(left != 0) != 0) redo |= 1u << (2 * nt + mt);
     }
   for (; redo != 0; redo &= redo - 1) {
     const int mt = __builtin_ctz(redo) & 1, nt = __builtin_ctz(redo) >> 1, v = vb + 32 * nt;
@@ -578,7 +594,9 @@ __global__ __launch_bounds__(256) void k_head_sum(HeadArgs a, int slices) {
 #pragma unroll 8
   for (int z = 0; z < slices; ++z) s += p[z * pitch];
   if constexpr (SPLIT) {
-    if (not_finite(s)) {
+    if (not_finite(s) && a.nan_rows[n] != 0) {
+      s = NAN;
+    } else if (not_finite(s)) {
       const float* x = a.act32 + (size_t)n * split_groups(a.D) * 8;
       s = 0.0f;
 #pragma unroll 8
@@ -648,10 +666,10 @@ HeadPlan head_plan(int N, int D, int V, int64_t ldw, int num_cu) {
   return best;
 }
 
-// The workspace: act in the product's layout, for k_head_split also in float32;
-// the partial sums.  Offsets in bytes.
+// The workspace: act in the product's layout; for k_head_split also in float32,
+// and the rows that hold a NaN; the partial sums.  Offsets in bytes.
 struct HeadWs {
-  size_t act32, part, bytes;
+  size_t act32, nan_rows, part, bytes;
 };
 
 HeadWs head_ws(const HeadPlan& p, int N, int D, int V) {
@@ -665,6 +683,7 @@ HeadWs head_ws(const HeadPlan& p, int N, int D, int V) {
   };
   HeadWs w{};
   w.act32 = take(split ? K * N * sizeof(float) : 0);
+  w.nan_rows = take(split ? rows * sizeof(int) : 0);
   w.part = take(p.slices > 1 ? (size_t)p.slices * N * V * sizeof(float) : 0);
   w.bytes = at;
   return w;
@@ -696,6 +715,7 @@ hipError_t launch_head(HeadArgs a, int num_cu, hipStream_t s) {
   const HeadWs ws = head_ws(p, a.N, a.D, a.V);
   char* base = static_cast<char*>(a.act);
   a.act32 = reinterpret_cast<float*>(base + ws.act32);
+  a.nan_rows = reinterpret_cast<int*>(base + ws.nan_rows);
   a.part = reinterpret_cast<float*>(base + ws.part);
   a.lda = (int64_t)((a.N + p.rows - 1) / p.rows) * p.rows;
   switch (p.rows) {

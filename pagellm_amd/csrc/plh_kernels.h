@@ -147,6 +147,7 @@ struct HeadArgs {
   void* act;          // workspace: the normalised rows in the product's operand layout
   int64_t lda;        // rows of act (whole row tiles)
   float* act32;       // workspace [N, D padded to whole stages]: the rows in float32 (k_head_split)
+  int* nan_rows;      // workspace [lda]: 1 for rows that hold a NaN (k_head_split)
   float* part;        // workspace [slices, N, V]: partial sums, with several slices of k
   int N, D, V;
 };

@@ -207,6 +207,27 @@ def test_many_rows_and_rows_of_lm_head_far_apart(N, V, ldw):
     assert bool(((got - a @ W.double()).abs() <= 1e-6 * (a.abs() @ W.double().abs())).all())
 
 
+@pytest.mark.parametrize("N,D,V", [(40, 64, 70000), (40, 1000, 333), (100, 1016, 70001), (200, 1000, 50257)])
+def test_a_nan_row_leaves_the_others_alone(N, D, V):
+    """One broken row of hidden states: its logits are NaN, and no tile of the
+    other rows is formed again (in another order of the sum: other bits)."""
+    import torch
+
+    print(f"[head] NaN row N={N} D={D} V={V}", flush=True)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(N)
+    W = 0.02 * torch.randn((D, V), generator=g, device="cuda")
+    h = torch.randn((N, D), generator=g, device="cuda")
+    norm = torch.ones(D, device="cuda")
+    ref = H.rms_norm_lm_head(h, norm, W, 1e-5).clone()
+    for bad in (float("nan"), float("inf")):
+        h[5, D // 2] = bad
+        got = H.rms_norm_lm_head(h, norm, W, 1e-5)
+        assert bool(got[5].isnan().all())
+        got[5] = ref[5]
+        assert torch.equal(got, ref)
+
+
 def test_tiny_rows_and_eps():
     """Rows of norm ~1e-3 (eps visible), an all-zero row (r = 1/sqrt(eps))."""
     h, norm, W = _case(3, 6, 96, 257, scale=1e-3)
