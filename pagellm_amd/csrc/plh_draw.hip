@@ -2,21 +2,25 @@
 // inverse-CDF draw from rows of non-negative weights.
 //
 // A row is cut into pieces of 512 tokens.  One pass over the row sums each
-// piece in float64 (a wave's piece is whole 16-byte loads of consecutive
-// tokens); the running piece totals, added in one fixed order, give W and the
-// first piece whose total exceeds u * W, and only that piece is read again for
-// the token.  float32 rows are widened exactly.
+// piece (a wave's piece is whole 16-byte loads of consecutive tokens); the
+// running piece totals give the total W and the first piece whose total exceeds
+// u * W, and only that piece is read again for the token.  float32 rows are
+// widened exactly.
 //
-//   k_draw_row    one workgroup per row, the piece sums in LDS: one launch;
-//   k_draw_parts  a workgroup per 16 384 tokens of a row, the piece sums in
-//   k_draw_pick   the workspace, then a wave per row: for long rows that are
-//                 too few to fill the chip one workgroup each.
+// Masses are added in fixed point, in units of 2^-62 of the power of two above
+// W (a scaling, exact, where a division by W rounds), so a total does not depend
+// on the order of its sum, and u times the total is exact; a piece's own mass is
+// summed in float64 first, but in a row of at most 8 pieces, which a wave each
+// keeps in registers.  How far a boundary between tokens lies from its exact
+// place (rms, in W; logits N(0, 2); masses divided by W in units of 2^-62 and a
+// rounded u * W / float64 throughout / here): 512 tokens 3.9e-17 / 7.4e-17 /
+// 1.1e-18, 4096 3.6e-17 / 7.6e-17 / 2.5e-18, 32 000 4.1e-17 / 7.1e-17 / 2.5e-17,
+// 152 064 3.9e-17 / 7.5e-17 / 2.4e-17.
 //
-// The float64 sums run in another order than numpy's cumsum, so the token
-// differs from the reference's only when u lies within ~1e-15 (relative) of a
-// CDF boundary.  Where rounding leaves the crossing just past the piece's end,
-// the piece's last token of positive weight is taken (a neighbour of the
-// boundary either way).
+// The token differs from the reference's (numpy's float64 cumsum) only when u
+// lies within ~1e-15 (relative) of a CDF boundary.  Where rounding leaves the
+// crossing just past the piece's end, the piece's last token of positive weight is
+// taken (a neighbour of the boundary either way).
 //
 // Bound by the read of the rows and, for a few dozen rows, by one workgroup's
 // latency chain (a load round trip, the piece sums, the reread).
@@ -79,25 +83,128 @@ __device__ __forceinline__ void sum_pieces(const TIn* p, int V, int s0, int s1, 
   }
 }
 
+// Whether a row of total mass W is drawn from: not without mass, or with more
+// than a double holds, or for a u past the end: the last id (sampling.py:98
+// clamps to V - 1).
+__device__ __forceinline__ bool drawable(double W, double u) {
+  return W > 0.0 && W <= 1.7976931348623157e308 && u < 1.0;
+}
+
+// Fixed-point masses in units of 2^-62 of the power of two above W.
+struct FxScale {
+  int shift;
+  __device__ __forceinline__ explicit FxScale(double W) : shift(62 - __builtin_amdgcn_frexp_exp(W)) {}
+  __device__ __forceinline__ uint64_t operator()(double w) const { return __double2ull_rn(ldexp(w, shift)); }
+};
+
+// floor(u * tot) for u < 1 (0 for u <= 0), exact: below tot.
+__device__ __forceinline__ uint64_t fx_target(double u, uint64_t tot) {
+  if (!(u > 0.0)) return 0;
+  const uint64_t m = (uint64_t)ldexp(__builtin_amdgcn_frexp_mant(u), 53);  // u = m 2^-s
+  const int s = 53 - __builtin_amdgcn_frexp_exp(u);                        // at least 53
+  const uint64_t hi = __umul64hi(m, tot), lo = m * tot;
+  if (s < 64) return (hi << (64 - s)) | (lo >> s);
+  return s < 128 ? hi >> (s - 64) : 0;
+}
+
+// The first token of piece s whose running mass exceeds t, INT_MAX where none
+// does; before: the running mass at the piece's start; x: the lane's tokens, as
+// load_piece lays them out.  last: the piece's last token of positive weight.
+template <typename TIn>
+__device__ __forceinline__ int pick_fx(const typename PieceGeo<TIn>::V (&x)[PieceGeo<TIn>::kLoads], int s,
+                                       const FxScale& fx, uint64_t before, uint64_t t, int* last) {
+  using G = PieceGeo<TIn>;
+  int hit = INT_MAX, pos = -1;
+#pragma unroll
+  for (int j = 0; j < G::kLoads; ++j) {
+    uint64_t w[G::kVW], ts = 0;
+#pragma unroll
+    for (int e = 0; e < G::kVW; ++e) ts += w[e] = fx(weight_of((double)x[j][e]));
+    const uint64_t incl = wave_scan_incl(ts, (uint64_t)0, OpAdd{});
+    uint64_t c = before + (incl - ts);
+    const int i0 = s * kPiece + (j * kWave + lane()) * G::kVW;
+#pragma unroll
+    for (int e = 0; e < G::kVW; ++e) {
+      c += w[e];
+      if (hit == INT_MAX && c > t) hit = i0 + e;
+      if (x[j][e] > TIn(0)) pos = i0 + e;
+    }
+    before += lane_value(incl, kWave - 1);
+  }
+  *last = wave_max(pos);
+  return wave_min(hit);
+}
+
 // The drawn token of a row whose n piece sums are sum(i); by one wave, every
 // lane alike.
 template <typename TIn, class Sum>
 __device__ __forceinline__ int pick_token(const TIn* p, int V, double u, const Sum& sum, int n) {
   using G = PieceGeo<TIn>;
   const double W = pieces_total(sum, n);
-  // no mass, or more than a double holds, or u past the end: the last id
-  // (sampling.py:98 clamps to V - 1)
-  if (!(W > 0.0) || W > 1.7976931348623157e308 || u >= 1.0) return V - 1;
-  const double t = fmax(u * W, 0.0);
-  const Crossing c = cross_pieces(sum, n, t);
+  if (!drawable(W, u)) return V - 1;
+  const FxScale fx(W);
+  uint64_t tot = 0;
+  for (int base = 0; base < n; base += kWave) tot += wave_sum(fx(sum(base + lane())));
+  const uint64_t t = fx_target(u, tot);
+  uint64_t run = 0, before = 0;
+  int piece = -1;
+  for (int base = 0; base < n && piece < 0; base += kWave) {
+    const uint64_t v = fx(sum(base + lane())), incl = run + wave_scan_incl(v, (uint64_t)0, OpAdd{});
+    const uint64_t over = __ballot(incl > t);
+    if (over != 0) {
+      const int k = __builtin_ctzll(over);
+      piece = base + k;
+      before = lane_value(incl - v, k);
+    }
+    run = lane_value(incl, kWave - 1);
+  }
   typename G::V x[G::kLoads];
-  load_piece(p, V, c.piece, x);
-  double w[G::kLoads][G::kVW];
+  load_piece(p, V, piece, x);
+  int last;
+  const int hit = pick_fx<TIn>(x, piece, fx, before, t, &last);
+  return hit != INT_MAX ? hit : last;
+}
+
+// The same for a row of at most kWaves pieces, one a wave, kept in registers;
+// by the whole workgroup.
+template <typename TIn>
+__device__ __forceinline__ void draw_short_row(const TIn* p, int V, double u, int32_t* out) {
+  using G = PieceGeo<TIn>;
+  __shared__ double sums[kWaves];
+  __shared__ uint64_t mass[kWaves];
+  const int w = uniform(wave());
+  typename G::V x[G::kLoads];
+  load_piece(p, V, w, x);  // zeros past the row
+  const double mine = wave_sum(lane_sum<TIn>(x));
+  if (lane() == 0) sums[w] = mine;
+  wg_barrier();
+  double W = 0.0;
+#pragma unroll
+  for (int i = 0; i < kWaves; ++i) W += sums[i];
+  if (!drawable(W, u)) {
+    if (threadIdx.x == 0) *out = V - 1;
+    return;
+  }
+  const FxScale fx(W);
+  uint64_t m = 0;
 #pragma unroll
   for (int j = 0; j < G::kLoads; ++j)
 #pragma unroll
-    for (int e = 0; e < G::kVW; ++e) w[j][e] = weight_of((double)x[j][e]);
-  return pick_in_piece<TIn>(c, t, w);
+    for (int e = 0; e < G::kVW; ++e) m += fx(weight_of((double)x[j][e]));
+  m = wave_sum(m);
+  if (lane() == 0) mass[w] = m;
+  wg_barrier();
+  uint64_t before = 0, tot = 0;
+#pragma unroll
+  for (int i = 0; i < kWaves; ++i) {
+    if (i == w) before = tot;
+    tot += mass[i];
+  }
+  const uint64_t t = fx_target(u, tot);
+  if (t < before || t - before >= m) return;  // uniform: one wave goes on
+  int last;
+  const int hit = pick_fx<TIn>(x, w, fx, before, t, &last);
+  if (lane() == 0) *out = hit;
 }
 
 template <typename TIn>
@@ -106,6 +213,10 @@ __global__ __launch_bounds__(kThreads) void k_draw_row(DrawArgs a) {
   const int row = blockIdx.x, n = (a.V - 1) / kPiece + 1, w = uniform(wave());
   const TIn* p = reinterpret_cast<const TIn*>(a.p) + (int64_t)row * a.ld;
   const double u = a.uniforms[row];
+  if (n <= kWaves) {  // the kernel's rows are all of V tokens: uniform
+    draw_short_row(p, a.V, u, a.out_ids + row);
+    return;
+  }
   int id;
   if (n <= kMaxPieces) {
     const int per = (n + kWaves - 1) / kWaves, s0 = min(w * per, n), s1 = min(s0 + per, n);

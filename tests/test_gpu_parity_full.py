@@ -217,3 +217,26 @@ def test_draw_under_graph_capture():
         ref = [oracle.draw(hp[b], float(hu[b])) for b in range(B)]
         assert ids.tolist() == ref == draw_batch(hp, hu).tolist()
     c.set_stream(None)
+
+
+@pytest.mark.parametrize("V", [65, 512, 4096])
+def test_draw_on_either_side_of_a_boundary(V):
+    """u at the two doubles next to a boundary of the CDF (taken from 64-bit
+    mantissas): the token on its side, unless the boundary is within 8 standard
+    deviations of the roundings of V masses to 2^-62 of the total (u times the
+    total, and the sums, are exact)."""
+    g = np.random.default_rng(V)
+    B = 64
+    p = _rows(g, 1, V, "softmax")[0]
+    c = np.cumsum(p.astype(np.longdouble))
+    c /= c[-1]
+    at = np.sort(g.choice(V - 1, B, replace=False))
+    u = np.concatenate([np.nextafter(c[at].astype(float), s) if s is not None else c[at].astype(float)
+                        for s in (None, 0.0, 1.0)])
+    u = u[(u > 0) & (u < 1)]
+    gap = np.abs(c[None, :] - u[:, None].astype(np.longdouble)).min(axis=1)
+    clear = gap > 8 * np.sqrt(V / 12) * 2.0 ** -62
+    assert clear.sum() > B
+    want = np.searchsorted(c, u.astype(np.longdouble), side="right")
+    ids = draw_batch(np.repeat(p[None], u.size, axis=0), u)
+    assert np.array_equal(ids[clear], want[clear])
