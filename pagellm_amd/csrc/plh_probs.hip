@@ -58,16 +58,23 @@ struct ProbsSmem {
 };
 
 // Workgroup reductions over 16 waves: each wave's value to LDS, one barrier,
-// every thread combines them in order; a second barrier frees the slots.
+// every thread combines them pairwise in one order; a second barrier frees the
+// slots.  Pairwise, because the last additions carry most of the rounding of a
+// float64 sum: the normaliser of 32 000 tokens is 7e-17 from exact (rms), 1.1e-16
+// with the waves added one after another.
 template <typename T, class Op>
 __device__ __forceinline__ T all_waves(T v, T* red, const Op& op) {
   if (lane() == 0) red[wave()] = v;
   __syncthreads();
-  T r = red[0];
+  T r[kPW];
 #pragma unroll
-  for (int w = 1; w < kPW; ++w) r = op(r, red[w]);
+  for (int w = 0; w < kPW; ++w) r[w] = red[w];
+#pragma unroll
+  for (int h = kPW / 2; h > 0; h >>= 1)
+#pragma unroll
+    for (int w = 0; w < h; ++w) r[w] = op(r[w], r[w + h]);
   __syncthreads();
-  return r;
+  return r[0];
 }
 
 // Exclusive scan of one value per thread.

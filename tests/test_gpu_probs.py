@@ -83,3 +83,26 @@ def test_probs_rows(V, dtype):
         c.sample(d["x"].ptr, _native.dtype_code(buf.dtype), V + 3, B, V, d["hi"].ptr, d["ho"].ptr, d["t"].ptr, d["k"].ptr,
                  d["p"].ptr, d["r"].ptr, d["u"].ptr, ids.ptr, None, 0)
         assert np.array_equal(ids.download(), out.download())
+
+
+@pytest.mark.parametrize("V", [8192, 32000])
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_rows_sum_to_one(V, dtype):
+    """The rows' exact sums are off by the normaliser's rounding and that of its
+    reciprocal (rms over the rows): pairwise sums over waves and lanes stay
+    within 1e-16, waves added one after another exceed it."""
+    g = np.random.default_rng(V)
+    B = 192
+    x = (2 * g.standard_normal((B, V))).astype(dtype)
+    print(f"[probs] sums V={V} {np.dtype(dtype).name}", flush=True)
+    c = _native.default_context()
+    c.set_stream(None)
+    t, k, p, r = _pack_params([SamplingParams()] * B)
+    d = {n: c.to_device(a) for n, a in dict(x=x, t=t, k=k, p=p, r=r, u=np.full(B, 0.5)).items()}
+    out, pr = c.empty((B,), np.int32), c.empty((B, V), np.float64)
+    c.sample(d["x"].ptr, _native.dtype_code(x.dtype), V, B, V, None, None, d["t"].ptr, d["k"].ptr, d["p"].ptr, d["r"].ptr,
+             d["u"].ptr, out.ptr, pr.ptr, 0)
+    off = pr.download().astype(np.longdouble).sum(axis=1) - 1
+    rms = float(np.sqrt(np.mean(off ** 2)))
+    print(f"[probs] rms {rms:.2e}", flush=True)
+    assert rms < 1e-16, rms
