@@ -179,7 +179,11 @@ int plh_penalize(plh_ctx* ctx, const void* x, int dtype, int64_t ld, int B, int 
  * draw(): src/pagellm/engine/sampling.py:94-98 for B rows of non-negative
  * weights p[b, :V] (any scale): first i with cumsum(p)[i] > u[b] * sum(p),
  * else V-1.  float32 rows are widened exactly and drawn in float64
- * arithmetic (the reference's probs() hands draw() float64 rows).
+ * arithmetic (the reference's probs() hands draw() float64 rows).  Rows of
+ * more than 40 000 tokens that are at most a quarter as many as the GPU's
+ * compute units, and rows of more than 1 048 576, use the context's workspace:
+ * such a call may allocate, and is ordered with the context's other workspace
+ * calls on whatever stream.  Others, and calls under graph capture, use none.
  */
 int plh_draw(plh_ctx* ctx, const void* p, int dtype, int64_t ld, int B, int V,
              const double* uniforms, int32_t* out_ids);

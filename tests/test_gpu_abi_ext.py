@@ -282,10 +282,10 @@ def test_workspace_calls_on_changing_streams():
 
 
 def test_workspace_users_interleaved_on_streams():
-    """plh_sample, plh_verify and plh_rmsnorm_lm_head share the context's
-    workspace (each grows it to its own size).  Interleaved over three
-    streams with no host wait between the calls, every result equals the
-    same call made alone on one stream."""
+    """plh_sample and plh_rmsnorm_lm_head, which share the context's workspace
+    (each grows it to its own size), and plh_verify at a size that needs none.
+    Interleaved over three streams with no host wait between the calls, every
+    result equals the same call made alone on one stream."""
     import torch
 
     from pagellm_amd import workloads
@@ -348,6 +348,75 @@ def test_workspace_users_interleaved_on_streams():
                 assert np.array_equal(r[0].download(), ref_t) and np.array_equal(r[1].download(), ref_n), i
             else:
                 assert np.array_equal(r.download(), ref_h), i
+    finally:
+        c.set_stream(None)
+        c.close()
+
+
+@pytest.mark.parametrize("order", ["dvsh", "vdhs", "shdv", "hsvd"])
+def test_every_workspace_user_interleaved_on_streams(order):
+    """All four users of the context's workspace, at sizes that use it: draws of
+    few long rows (d) and verify of longer rows (v), two launches each, sampling
+    (s) and the logits product (h).  A fresh context per order, so that each
+    grows the workspace behind another one's queued call; every call moves to
+    the next of three streams, twice round, with no host wait."""
+    import torch
+
+    from pagellm_amd import workloads
+
+    g = np.random.default_rng(29)
+    zw = workloads.zipf32k()
+    Vd, Bd = 152064, 16
+    pd, ud = g.random((Bd, Vd)), g.random(Bd)
+    Bv, k, Vv = 8, 3, 50257
+    p, q = g.random((Bv, k + 1, Vv)), g.random((Bv, k, Vv))
+    p, q = p / p.sum(-1, keepdims=True), q / q.sum(-1, keepdims=True)
+    draft = g.integers(0, Vv, (Bv, k)).astype(np.int32)
+    acc_u, res_u = g.random((Bv, k)) * 0.9, g.random(Bv)
+    N, D, Vh = 40, 512, 3000  # slices of k
+    h = g.normal(0, 1, (N, D)).astype(np.float32)
+    norm = g.normal(1, 0.1, D).astype(np.float32)
+    wt = g.normal(0, 0.05, (D, Vh)).astype(np.float32)
+
+    def inputs(c):
+        return {n: c.to_device(a) for n, a in dict(pd=pd, ud=ud, p=p, q=q, d=draft, a=acc_u, w=res_u, h=h, n=norm,
+                                                   wt=wt).items()}
+
+    def draw_call(c, d):
+        out = c.empty((Bd,), np.int32)
+        c.draw(d["pd"].ptr, _native.PLH_F64, Vd, Bd, Vd, d["ud"].ptr, out.ptr)
+        return (out,)
+
+    def verify_call(c, d):
+        tok, nacc = c.empty((Bv, k + 1), np.int32), c.empty((Bv,), np.int32)
+        c.verify(d["p"].ptr, d["q"].ptr, _native.PLH_F64, Bv, k, Vv, d["d"].ptr, d["a"].ptr, d["w"].ptr, 0, tok.ptr,
+                 nacc.ptr)
+        return tok, nacc
+
+    def head_call(c, d):
+        out = c.empty((N, Vh), np.float32)
+        c.rmsnorm_lm_head(d["h"].ptr, D, N, D, d["n"].ptr, 1e-6, d["wt"].ptr, Vh, Vh, out.ptr, Vh)
+        return (out,)
+
+    call = {"d": draw_call, "v": verify_call, "h": head_call, "s": lambda c, d: (_launch_rows(c, zw, rows=48),)}
+    c = _native.Context(0)
+    try:
+        d = inputs(c)
+        ref = {o: [a.download() for a in call[o](c, d)] for o in "dvhs"}
+    finally:
+        c.close()
+    c = _native.Context(0)
+    try:
+        d = inputs(c)
+        streams = [torch.cuda.Stream().cuda_stream, None, torch.cuda.Stream().cuda_stream]
+        got = []
+        for i, o in enumerate(order + order[::-1]):
+            c.set_stream(streams[i % 3])
+            got.append((o, call[o](c, d)))
+        torch.cuda.synchronize()
+        for i, (o, r) in enumerate(got):
+            for a, b in zip(r, ref[o]):
+                assert np.array_equal(a.download(), b), (i, o)
     finally:
         c.set_stream(None)
         c.close()
