@@ -11,10 +11,13 @@ rtol = atol = 1e-4 (``tests/unit/test_model.py:55``)."""
 
 from __future__ import annotations
 
+import ctypes
+
 import numpy as np
 import pytest
 
 import oracle
+from pagellm_amd import _native
 from pagellm_amd import head as H
 
 pytestmark = pytest.mark.gpu
@@ -51,16 +54,26 @@ def test_head_matches_oracle(N, D, V):
     np.testing.assert_allclose(got, ref, rtol=1e-4, atol=1e-4)
 
 
-# (1, 16, 17, 32): the few-rows kernels; 33 on: the split kernels, with
-# ragged and whole row tiles.  A (D, V) pair reaches, as N grows, one and
-# several slices of k and every tile height.
+def _plan(N, D, V):
+    """(rows per workgroup, slices of k) that the library picks for the device."""
+    import torch
+
+    f = ctypes.CDLL(str(_native.LIB_PATH))["_ZN3plh9head_planEiiili"]  # plh::head_plan
+    f.restype, f.argtypes = ctypes.c_uint64, [ctypes.c_int] * 3 + [ctypes.c_int64, ctypes.c_int]
+    r = f(N, D, V, V, torch.cuda.get_device_properties(0).multi_processor_count)
+    return r & 0xffffffff, r >> 32
+
+
+# (1, 16, 17, 32): the few-rows kernels, in one and several slices of k; 33 on:
+# the split kernels, in tiles of 64 rows (and at 70 000 columns of 128), with
+# ragged and whole row tiles.  test_tile_plans has the other plans.
 @pytest.mark.parametrize("N", [1, 16, 17, 32, 33, 64, 65, 129, 256])
 @pytest.mark.parametrize("D,V", [
     (8, 127),     # one column short of a workgroup; k ends in a ragged group (16 rows) or a whole one (32)
     (128, 128),   # one workgroup, whole groups and stages
     (129, 257),   # the last workgroup's columns overlap the one's before; one k past the whole groups
     (1000, 333),  # several slices of k, the last one ragged
-    (40, 70000),  # enough columns for every tile height in one slice
+    (40, 70000),  # enough columns for one slice at every N
 ])
 def test_row_counts_and_edges(N, D, V):
     """Every kernel on W, h and out rows of odd strides (no 16-byte alignment
@@ -226,6 +239,29 @@ def test_a_nan_row_leaves_the_others_alone(N, D, V):
         assert bool(got[5].isnan().all())
         got[5] = ref[5]
         assert torch.equal(got, ref)
+
+
+# Every tile height in one and several slices, rows, k and columns all ragged.
+TILES = [
+    (45, 203, 50257, 64, 1),
+    (45, 1015, 333, 64, 16),
+    (100, 63, 70001, 128, 1),
+    (100, 1015, 70001, 128, 2),
+    (250, 203, 70001, 256, 1),
+    (255, 1999, 20001, 256, 2),
+]
+
+
+@pytest.mark.parametrize("N,D,V,rows,slices", TILES)
+def test_tile_plans(N, D, V, rows, slices):
+    assert _plan(N, D, V) == (rows, slices)  # else this case tests another kernel than it names
+    test_row_counts_and_edges(N, D, V)
+
+
+@pytest.mark.parametrize("N,D,V,rows,slices", TILES)
+def test_values_at_the_ends_of_float32_in_every_tile(N, D, V, rows, slices):
+    assert _plan(N, D, V) == (rows, slices)
+    test_values_at_the_ends_of_float32(N, D, V)
 
 
 def test_tiny_rows_and_eps():
