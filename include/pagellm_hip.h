@@ -88,7 +88,8 @@ int plh_set_option(plh_ctx* ctx, int option, int64_t value);
 int plh_fallback_rows(plh_ctx* ctx, int64_t* out);
 /* While PLH_OPT_KERNEL_TIMING is on: device time of the fast path's
  * streaming kernel and merge kernel summed over the plh_sample calls made
- * since the last read, and their count.  Waits for those calls, then
+ * since the last read, and their count (calls of one launch, and plh_verify's,
+ * too: their only or first kernel counts as the streaming one).  Waits for those calls, then
  * resets.  No reference counterpart (measurement only). */
 int plh_kernel_times(plh_ctx* ctx, double* stream_ms, double* merge_ms, int64_t* calls);
 
@@ -232,11 +233,18 @@ int plh_append_ids(plh_ctx* ctx, int32_t* slab, const int64_t* pos, const int32_
  * place:
  *   r_n = 1 / sqrt(mean_d(h[n, d]^2) + eps)      (float32, eps as a float32)
  *   out[n, v] = sum_d ((h[n, d] * r_n) * norm[d]) * W[d, v]
- * for n < N, v < V, with the products and sums in float32 on the matrix
- * cores.  h [N, ldh], norm [D], W [D, ldw] (row-major: the reference's
- * [D, V] lm_head) and out [N, ldo] are float32 device pointers; the
- * normalised rows live in the context's workspace.  Ordered on the
- * context's stream.
+ * for n < N, v < V.  Up to 32 rows (and sums of fewer than 4 products) are
+ * formed on the fp32 matrix cores; more rows from six bf16 products per float32
+ * product, summed in float32, which is no further from the exact sum (the rest
+ * of a product is below 2^-24 of its operands' powers of two).  Sums of 2^34 and
+ * more, infinities and NaN come out as float32 products give them.
+ * The order of a sum depends on (N, D, V, ldw) and the device: equal calls give
+ * equal bits, but a row's logits may differ in their last bits with the number
+ * of rows beside it.
+ * h [N, ldh], norm [D], W [D, ldw] (row-major: the reference's [D, V] lm_head)
+ * and out [N, ldo] are float32 device pointers; the normalised rows, and partial
+ * sums where k is cut into slices, live in the context's workspace.  Ordered on
+ * the context's stream.
  */
 int plh_rmsnorm_lm_head(plh_ctx* ctx, const float* h, int64_t ldh, int N, int D, const float* norm, double eps,
                         const float* W, int64_t ldw, int V, float* out, int64_t ldo);

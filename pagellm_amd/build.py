@@ -20,7 +20,6 @@ CSRC = PKG / "csrc"
 OUT = PKG / "libpagellm_hip.so"
 BUILD = PKG / "_build"
 SOURCES = ["plh_sample.hip", "plh_small.hip", "plh_probs.hip", "plh_draw.hip", "plh_verify.hip", "plh_head.hip", "plh_api.hip"]
-HEADERS = ["plh_device.h", "plh_pipeline.h", "plh_kernels.h"]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = os.environ.get("PLH_OFFLOAD_ARCH", "gfx950")

@@ -3,13 +3,19 @@
 // (src/pagellm/model/transformer.py:79-82, :271), in float32 as the
 // reference computes it, written straight into the sampler's logits buffer.
 //
-// Two launches: a prep kernel (one workgroup per row: RMSNorm with numpy's
-// float32 steps, and act = (h * r) * norm in the layout the product reads),
-// then the product:
+// Two launches, or three: a prep kernel (one workgroup per row: RMSNorm with
+// numpy's float32 steps, and act = (h * r) * norm in the layout the product
+// reads), the product, and where k is cut into slices their sum:
 //
-//   k_head_skinny   at most 32 rows: one read of W, fp32 matrix cores
+//   k_head_skinny   at most 32 rows, or sums of a few products: one read of W,
+//                   fp32 matrix cores
 //   k_head_split    more rows: float32 products on the bf16 matrix cores,
 //                   each operand split exactly into three bf16 parts
+//   k_head_sum      the slices' partial sums
+//
+// The order of a sum depends on N, D, V, ldw and the number of CUs (head_plan),
+// not on the data: equal calls give equal bits, but a row's last bits may change
+// with the number of rows beside it.
 #include "plh_device.h"
 #include "plh_kernels.h"
 
@@ -582,8 +588,8 @@ k_head_split(HeadArgs a) {
 
 // ------------------------------------------------------------ slices of k
 //
-// out = the slices' partial sums added in order.  SPLIT: an element that the
-// bf16 parts cannot carry is formed again in float32.
+// out = the slices' partial sums added in order.  SPLIT: they are scaled, and an
+// element that the bf16 parts cannot carry is formed again in float32.
 template <bool SPLIT>
 __global__ __launch_bounds__(256) void k_head_sum(HeadArgs a, int slices) {
   const int v = blockIdx.x * 256 + threadIdx.x, n = blockIdx.y;
@@ -619,8 +625,7 @@ struct HeadPlan {
 // times k steps times one step, but at least the read of W, plus the partial
 // sums' way through the caches.  The steps were measured at N 8 to 256 over
 // 4096 x 1000 (4 to 16 workgroups: a step's latency) and 4096 x 128 256 (every
-// CU at work: its throughput); over 54 sizes of (N, D, V) the plan this picks
-// is within 2% of the fastest of 20 in 46 of them, and within 16% in all.
+// CU at work: its throughput).
 double plan_us(const HeadPlan& p, int N, int D, int V, int num_cu) {
   const double w_bytes = 4.0 * D * V, rows = (N + p.rows - 1) / p.rows;
   double us;
@@ -647,7 +652,8 @@ double plan_us(const HeadPlan& p, int N, int D, int V, int num_cu) {
 // the read of W, not by the matrix cores (at 157 TFLOP/s 32 rows take half of
 // W's time in HBM), and k_head_skinny reads W at the rate of a copy; 33 rows
 // on would read it twice there (4096 x 128 256: 720 us for 17 rows in two tiles
-// of 16, 410 us in one of 32).  Slices fill the chip where the columns alone
+// of 16, 410 us in one of 32).  Sums of fewer than kSplitMinD products go there for
+// their precision (the table at k_head_split).  Slices fill the chip where the columns alone
 // do not (4096 x 1000, 8 rows: 44 us in one slice, 15 us in 16).
 HeadPlan head_plan(int N, int D, int V, int64_t ldw, int num_cu) {
   const bool skinny = N <= 32 || D < kSplitMinD || ldw > kSplitMaxLdw;

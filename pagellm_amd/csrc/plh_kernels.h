@@ -188,8 +188,9 @@ VerifyWs verify_ws_layout(void* base, int B, int V);
 // `between`, when not null, is recorded on s between the two launches.
 hipError_t launch_verify(const VerifyArgs& a, const VerifyWs& ws, bool f64, hipStream_t s,
                          hipEvent_t between = nullptr);
-// Logits producer: workspace bytes (the normalised rows) and the two
-// launches (RMSNorm, then the MFMA product into out).
+// Logits producer: workspace bytes (the normalised rows, and the partial sums of
+// several slices of k) and the launches (RMSNorm, the MFMA product into out or
+// the partial sums, and with slices their sum).
 size_t head_ws_bytes(int N, int D, int V, int64_t ldw, int num_cu);
 hipError_t launch_head(HeadArgs a, int num_cu, hipStream_t s);
 hipError_t launch_append(int32_t* slab, const int64_t* pos, const int32_t* ids, int n, hipStream_t s);

@@ -4,8 +4,11 @@
 self.w["lm_head"]`` (``src/pagellm/model/transformer.py:271``, ``rms_norm``
 at ``:79-82``), in the model's dtype, float32 by default
 (``init_weights``, ``:184-197``).  :func:`rms_norm_lm_head` computes the same
-float32 logits with ``plh_rmsnorm_lm_head`` (fp32 matrix cores) and writes
-them where the sampler reads them, so that a step's logits never leave HBM:
+float32 logits with ``plh_rmsnorm_lm_head`` (up to 32 rows on the fp32 matrix
+cores, more on the bf16 ones with each operand split into three parts, no
+further from the exact sums) and writes them where the sampler reads them, so
+that a step's logits never leave HBM.  A row's last bits may depend on the
+number of rows in the call, which picks the order of its sums:
 
     head = LogitsHead(w["norm"], w["lm_head"], cfg.norm_eps)   # weights resident
     ids = sampler.sample(head(h), params, rngs, keys)           # no host copy
