@@ -738,7 +738,7 @@ def bench_verify(steps: int = 50, warmup: int = 5) -> dict:
         ctx.kernel_times()
         for i in range(steps):
             step(i)
-        kernel_ms, _, calls = ctx.kernel_times()  # one launch: all of it before the event between two
+        kernel_ms, _, calls = ctx.kernel_times()  # one launch (and the events' own cost)
         ctx.set_kernel_timing(False)
     n = nacc.cpu().numpy()
     nbytes = int(sum(16 * (min(int(s) + 1, k)) + (16 * V if s < k else 8 * V) for s in n))
