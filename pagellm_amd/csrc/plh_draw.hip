@@ -24,8 +24,8 @@
 //
 // Bound by the read of the rows and, for a few dozen rows, by one workgroup's
 // latency chain (a load round trip, the piece sums, the reread).
-// 64 x 32 000 float64: 39.9 -> 6.4 us against three passes over the row with a
-// float64 division per token; 512 x 152 064: 108 us, 5.8 TB/s.
+// 64 x 32 000 float64: 39.9 -> 6.3 us against three passes over the row with a
+// float64 division per token; 512 x 152 064: 106 us, 5.9 TB/s.
 #include "plh_device.h"
 #include "plh_kernels.h"
 #include "plh_pieces.h"
@@ -140,11 +140,14 @@ __device__ __forceinline__ int pick_fx(const typename PieceGeo<TIn>::V (&x)[Piec
 template <typename TIn, class Sum>
 __device__ __forceinline__ int pick_token(const TIn* p, int V, double u, const Sum& sum, int n) {
   using G = PieceGeo<TIn>;
-  const double W = pieces_total(sum, n);
+  double W = 0.0;  // sets the scale only: any order will do
+  for (int base = 0; base < n; base += kWave) W += sum(base + lane());
+  W = wave_sum(W);
   if (!drawable(W, u)) return V - 1;
   const FxScale fx(W);
   uint64_t tot = 0;
-  for (int base = 0; base < n; base += kWave) tot += wave_sum(fx(sum(base + lane())));
+  for (int base = 0; base < n; base += kWave) tot += fx(sum(base + lane()));
+  tot = wave_sum(tot);
   const uint64_t t = fx_target(u, tot);
   uint64_t run = 0, before = 0;
   int piece = -1;
