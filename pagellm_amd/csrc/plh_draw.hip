@@ -87,7 +87,7 @@ __device__ __forceinline__ void sum_pieces(const TIn* p, int V, int s0, int s1, 
 // than a double holds, or for a u past the end: the last id (sampling.py:98
 // clamps to V - 1).
 __device__ __forceinline__ bool drawable(double W, double u) {
-  return W > 0.0 && W <= 1.7976931348623157e308 && u < 1.0;
+  return W > 0.0 && W <= 1.7976931348623157e308 && !(u >= 1.0);
 }
 
 // Fixed-point masses in units of 2^-62 of the power of two above W.
@@ -97,7 +97,7 @@ struct FxScale {
   __device__ __forceinline__ uint64_t operator()(double w) const { return __double2ull_rn(ldexp(w, shift)); }
 };
 
-// floor(u * tot) for u < 1 (0 for u <= 0), exact: below tot.
+// floor(u * tot) for u < 1 (0 for u <= 0 and NaN), exact: below tot.
 __device__ __forceinline__ uint64_t fx_target(double u, uint64_t tot) {
   if (!(u > 0.0)) return 0;
   const uint64_t m = (uint64_t)ldexp(__builtin_amdgcn_frexp_mant(u), 53);  // u = m 2^-s

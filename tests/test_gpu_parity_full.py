@@ -240,3 +240,13 @@ def test_draw_on_either_side_of_a_boundary(V):
     want = np.searchsorted(c, u.astype(np.longdouble), side="right")
     ids = draw_batch(np.repeat(p[None], u.size, axis=0), u)
     assert np.array_equal(ids[clear], want[clear])
+
+
+@pytest.mark.parametrize("V", [300, 5000, 50257])
+def test_draw_uniforms_outside_the_unit_interval(V):
+    """u past the end takes the last id, u below 0 (and NaN) the first token of
+    positive weight: in registers, in one launch and in two."""
+    p = np.ones((4, V))
+    p[:, :7] = 0
+    ids = draw_batch(p, np.array([-0.5, np.nan, 1.0, 3.0]))
+    assert ids.tolist() == [7, 7, V - 1, V - 1]
